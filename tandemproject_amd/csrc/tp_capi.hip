@@ -363,12 +363,23 @@ size_t col_block_doubles(const int *L) {
 }
 
 // default chunk count of lines of L points: the fewest chunks (a power of
-// two) whose length stays within 24 points (registers for 4+ waves per SIMD),
-// else within 32; 0 (the sequential kernel) if none fits
-int col_default(int L) {
-  for (int lim : {24, 32})
-    for (int P : kColDefault)
-      if ((L + P - 1) / P <= lim) return P;
+// two, so that a compute unit's four SIMDs hold whole workgroups) whose length
+// stays within a limit; 0 (the sequential kernel) if none fits.  The limits,
+// from launches of 4 and 5 fields (us; L = 22 and 95 of a 1 M-point case, the
+// others of 9 M and 20 M points):
+//   L = 22:  1 chunk 33.5 / 41.9,  2 chunks 29.8 / 37.1,  4 chunks 32.6 / 43.9
+//   L = 48:  2 chunks 91 / 141,    4 chunks 96 / 151;  with closure faces, whose
+//            sums take registers:  2 chunks 397 / 672,  4 chunks 373 / 572
+//   L = 95:  4 chunks 24.0 / 35.5, 8 chunks 30.0 / 43.7
+//   L = 128: 4 chunks 41.0 / 44.7, 8 chunks 45.4 / 50.0
+//   L = 201: 8 chunks 300 / 558,   16 chunks 577 / 794
+//   L = 256: 8 chunks 78 / 88,     16 chunks 87 / 109
+// (up to 8 chunks two or more workgroups share a compute unit, one loading
+// while another sweeps; with 9 to 16 it holds one).
+int col_default(int L, bool closure) {
+  const int most[] = {8, closure ? 32 : 48, 128, 256, 512};
+  for (int i = 0; i < 5; i++)
+    if (L <= most[i]) return kColDefault[i];
   return 0;
 }
 
@@ -691,12 +702,14 @@ void drop_graph(tp_context *c) {
   if (c->graph) { (void)hipGraphDestroy(c->graph); c->graph = nullptr; }
 }
 
+int block_default(const Block &b, int d) { return col_default(b.L[d], b.ndf[d][0] || b.ndf[d][1]); }
+
 // chunks per line of block g's line solves in direction d, kind: the tuned
 // count of its line-length class if that fits its lines, else the requested
 // count if it fits, else the default (0: the sequential kernel)
 int block_chunks(const tp_context *c, int g, int d, int kind) {
   const int L = c->blocks[g].L[d];
-  const int def = col_default(L);
+  const int def = block_default(c->blocks[g], d);
   auto fits = [&](int P) { return P == 0 || col_chunk(L, P) != 0; };
   const int t = c->tuned[d][kind][col_class(def)];
   if (t >= 0 && fits(t)) return t;
@@ -2392,7 +2405,7 @@ int32_t tp_autotune(tp_context *c, int32_t reps, int32_t *chosen, double *us) {
     for (int kind = 0; kind < 2 && !rc; kind++) {
       // the line-length classes present, each tuned in turn with the others fixed
       bool present[kNClass] = {false};
-      for (const Block &b : c->blocks) present[col_class(col_default(b.L[d]))] = true;
+      for (const Block &b : c->blocks) present[col_class(block_default(b, d))] = true;
       float bestms = 1e30f;
       for (int cls = 0; cls < kNClass && !rc; cls++) {
         if (!present[cls]) continue;
@@ -2402,7 +2415,7 @@ int32_t tp_autotune(tp_context *c, int32_t reps, int32_t *chosen, double *us) {
           const int P = pi < 0 ? 0 : kColP[pi];   // 0: the sequential kernel
           bool ok = true;
           for (const Block &b : c->blocks)
-            if (col_class(col_default(b.L[d])) == cls && P && !col_chunk(b.L[d], P)) ok = false;
+            if (col_class(block_default(b, d)) == cls && P && !col_chunk(b.L[d], P)) ok = false;
           if (!ok) continue;
           c->tuned[d][kind][cls] = P;
           if ((rc = regroup(c))) break;
@@ -2833,7 +2846,7 @@ int field_prepare(int32_t lxi, int32_t let, int32_t lze, const int32_t *nbc2, in
   f.periodic = nbc2[0] == 45;
   if (f.L < (f.periodic ? LMD + 2 : 7))
     return fail(TP_E_LAYOUT, "tp_field_deriv: lines of " + std::to_string(f.L) + " points are too short");
-  f.P = col_default(f.L);
+  f.P = col_default(f.L, f.periodic);
   if (!f.P) return fail(TP_E_SIZE, "tp_field_deriv: lines longer than 512 points need a context (tp_deriv)");
   f.C = col_capacity((f.L + f.P - 1) / f.P);
   std::memset(&f.blk, 0, sizeof(Block));
