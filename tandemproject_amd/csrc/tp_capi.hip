@@ -724,15 +724,57 @@ void choose_lines(tp_context *c) {
     const auto &src = c->bsrc[g];
     for (int d = 0; d < 3; d++)
       for (int kind = 0; kind < 2; kind++) {
-        const int ci = col_class(block_chunks(c, (int)g, d, kind)) - 1;
+        const int P = block_chunks(c, (int)g, d, kind), ci = col_class(P) - 1;
+        c->blocks[g].colP[d][kind] = P;
         c->blocks[g].col[d][kind] =
             ci < 0 ? nullptr : c->cases[src.first].coltab[src.second][(d * 2 + kind) * kNColP + ci];
       }
   }
 }
 
+// Groups share a launch, at the largest chunk count and capacity among them,
+// while together they fill the GPU's 4096 wave slots (256 compute units x 16
+// waves of up to 128 registers) at most 8 times at five fields a launch: a
+// block's lines keep their own chunk count (Block::colP, the launch's further
+// waves only take part in the barriers and the stores) and capacity padding is
+// exact, so every result stays the same bits.  A launch of its own costs a
+// small group its latency and a nearly empty last round: the xi derivatives of a
+// 1 M-point case took 22 + 23 us as two launches and 33 us as one, those of
+// 208 k points 14 + 15 and 18 us; eight cases of 4.2 M points in all took 7.16 ms
+// a step with the limit at 1 or 2 times the slots and 6.96 with 8 (cases of 0.6,
+// 1 and 9 M points the same within their noise).  Groups of one chunk count
+// also join a larger group of that count.
+constexpr long long kSlots = 4096;
+void merge_groups(std::vector<ColGroup> &groups, std::vector<std::vector<Work>> &works) {
+  auto waves = [&](size_t k, int P) { return 5LL * P * (long long)works[k].size(); };
+  auto join = [&](size_t to, size_t k) {
+    ColGroup &a = groups[to], &b = groups[k];
+    a.P = std::max(a.P, b.P);
+    a.C = std::max(a.C, b.C);
+    a.closure = a.closure || b.closure;
+    a.npts += b.npts;
+    works[to].insert(works[to].end(), works[k].begin(), works[k].end());
+    groups.erase(groups.begin() + k);
+    works.erase(works.begin() + k);
+  };
+  for (bool again = true; again;) {
+    again = false;
+    for (size_t i = 0; i < groups.size() && !again; i++)
+      for (size_t k = 0; k < groups.size() && !again; k++) {
+        if (i == k || !groups[i].P || !groups[k].P || waves(k, groups[k].P) > waves(i, groups[i].P)) continue;
+        const int P = std::max(groups[i].P, groups[k].P);
+        const bool both = waves(i, P) + waves(k, P) <= 8 * kSlots;
+        const bool tail = groups[i].P == groups[k].P && groups[k].C <= groups[i].C && waves(k, P) <= kSlots;
+        if (both || tail) {
+          join(i, k);
+          again = true;
+        }
+      }
+  }
+}
+
 // line-solve launches over the global blocks gs: one per distinct chunk
-// count and chunk capacity of each direction and kind
+// count and chunk capacity of each direction and kind, small ones merged
 int make_groups(tp_context *c, const std::vector<int> &gs, Mem &m, ListSet &L) {
   for (int d = 0; d < 3; d++)
     for (int kind = 0; kind < 2; kind++) {
@@ -761,6 +803,7 @@ int make_groups(tp_context *c, const std::vector<int> &gs, Mem &m, ListSet &L) {
         for (int q = 0; q < nlines; q += step) works[k].push_back({g, q, std::min(step, nlines - q), d});
         groups[k].npts += b.N;
       }
+      merge_groups(groups, works);
       // a block and its neighbour across the end face of a closure (the two
       // halves of a split line) interleave their work items, so that the line
       // solves that form their closure sums from each other's lines run side
@@ -799,6 +842,13 @@ int make_groups(tp_context *c, const std::vector<int> &gs, Mem &m, ListSet &L) {
       L.cg[d][kind] = std::move(groups);
     }
   return 0;
+}
+
+// the chunk count that covers the most points (0: the sequential kernel)
+int top_chunks(const tp_context *c, int d, int kind) {
+  long long n[17] = {0};
+  for (const Block &b : c->blocks) n[b.colP[d][kind]] += b.N;
+  return (int)(std::max_element(n, n + 17) - n);
 }
 
 // rebuild the line-solve launches of the linked blocks after the chunk
@@ -2430,12 +2480,7 @@ int32_t tp_autotune(tp_context *c, int32_t reps, int32_t *chosen, double *us) {
       if ((rc = regroup(c))) break;
       float ms = 0;
       if ((rc = timed(d, kind, &ms))) break;
-      // report the chunk count that covers the most points
-      long long top = -1;
-      int P = 0;
-      for (const ColGroup &g : c->L.cg[d][kind])
-        if (g.npts > top) { top = g.npts; P = g.P; }
-      if (chosen) chosen[d * 2 + kind] = P;
+      if (chosen) chosen[d * 2 + kind] = top_chunks(c, d, kind);
       if (us) us[d * 2 + kind] = 1e3 * ms / reps;
     }
   }
@@ -2449,14 +2494,7 @@ int32_t tp_autotune(tp_context *c, int32_t reps, int32_t *chosen, double *us) {
 
 int32_t tp_col_config(tp_context *c, int32_t *chunks6) {
   if (!c || !chunks6) return fail(TP_E_ARG, "null argument");
-  for (int i = 0; i < 6; i++) {
-    long long top = -1;
-    int P = 0;
-    if (!c->exact_lines)
-      for (const ColGroup &g : c->L.cg[i / 2][i % 2])
-        if (g.npts > top) { top = g.npts; P = g.P; }
-    chunks6[i] = P;
-  }
+  for (int i = 0; i < 6; i++) chunks6[i] = c->exact_lines ? 0 : top_chunks(c, i / 2, i % 2);
   return 0;
 }
 
@@ -2863,6 +2901,7 @@ int field_prepare(int32_t lxi, int32_t let, int32_t lze, const int32_t *nbc2, in
     b.ncd[d][s] = f.periodic ? 0 : -1;
   }
   b.cs = 0;
+  b.colP[d][0] = f.P;
   b.rr = const_cast<double *>(src);   // read as rr(:,1) ...
   b.de = dst;                         // ... written as de(:,1)
   // coefficients: the derivative's closure rows, src/Main3D.f90:71-73, 309-312

@@ -288,7 +288,8 @@ __global__ void __launch_bounds__(1024) k_col(LineArgs a) {
   const Block &b = a.blocks[w.blk];
   const CaseCoef &c = a.coef[b.cs];
   const int L = b.L[D];
-  const int P = blockDim.x >> 6;
+  const int P = b.colP[D][KIND];                  // chunks of this block's lines
+  const int PL = blockDim.x >> 6;                 // waves of the launch, at least P
   const int p = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   const int Cl = (L + P - 1) / P;
@@ -305,10 +306,10 @@ __global__ void __launch_bounds__(1024) k_col(LineArgs a) {
   double *dst = field_ptr(b, a.out_arr, a.out_col + fi * a.out_step);
   const double *rcv = b.recv[D] + (size_t)fi * 6 * b.F[D];
   const int mcap = a.m > 0 ? a.m + fi : 0;
-  double2 *pairA = reinterpret_cast<double2 *>(lds);      // [P][64] carry-map inputs
-  double2 *pairB = pairA + P * 64;                        // [P][64] pairs handed along a chain
-  double *fl = reinterpret_cast<double *>(pairB + P * 64) + p * 192;   // [P][192] chunk factors
-  double *tr = reinterpret_cast<double *>(pairB + P * 64) + P * 192 + p * (8 * COL_TR);
+  double2 *pairA = reinterpret_cast<double2 *>(lds);      // [PL][64] carry-map inputs
+  double2 *pairB = pairA + PL * 64;                       // [PL][64] pairs handed along a chain
+  double *fl = reinterpret_cast<double *>(pairB + PL * 64) + p * 192;  // [PL][192] chunk factors
+  double *tr = reinterpret_cast<double *>(pairB + PL * 64) + PL * 192 + p * (8 * COL_TR);
   const double *T = b.col[D][KIND];
   const double mapf = T[lane], mapb = T[64 + lane];   // carry maps of all chunks
   ChunkLU f;
@@ -596,7 +597,7 @@ __global__ void __launch_bounds__(1024) k_col(LineArgs a) {
   // pieces (8 rows x 8 points) would straddle 64-byte write granules.
   const int pitch = L + 1;
   int R = 64;
-  while (R >= 8 && R * pitch > col_lds_doubles(0, P)) R >>= 1;
+  while (R >= 8 && R * pitch > col_lds_doubles(0, PL)) R >>= 1;
   if (D == 0 && R >= 8) {
     double *tile = lds;
     __syncthreads();

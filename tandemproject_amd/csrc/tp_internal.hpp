@@ -99,6 +99,7 @@ struct Block {
   double *snor;               // [3][nsurf] unit normals into the fluid (walldir)
   double *sst;                // [3][nsurf] previous sampled p, trapezoid integrals of p and p^2
   const double *col[3][2];    // chunked-solver carry maps per direction, kind (deriv, filter)
+  int colP[3][2];             // chunks per line they are for (0: the sequential kernel)
 };
 
 // array ids exposed through the C ABI (order shared with include/tandem_hip.h)
