@@ -474,7 +474,7 @@ struct ColGroup {
 };
 
 struct ListSet {
-  DevList points, sponge, force, lines[3], exch, gprep, gapply[3], gcopy, wall, acap, aapply[3], normals;
+  DevList points, sponge, force, lines[3], exch, gprep, gapply[3], wall, acap, normals;
   DevList surf;                     // wall-surface points, 256 per item
   std::vector<ColGroup> cg[3][2];   // line-solve launches per direction and kind
   std::vector<int> wr;   // first point-work item of each linked case, then the end
@@ -978,7 +978,6 @@ void enqueue_sponge(tp_context *c) {
 void enqueue_gcbc(tp_context *c) {
   const StageArgs a = base_args(c);
   run_faces(c, c->L.gprep, FK_GCBC_PREP, a, K_GCBC);
-  run_faces(c, c->L.gcopy, FK_COPY, a, K_GCBC);
   for (int d = 0; d < 3; d++) run_faces(c, c->L.gapply[d], d == 0 ? FK_GCBC_APPLY_XI : FK_GCBC_APPLY, a, K_GCBC);
 }
 
@@ -1013,9 +1012,8 @@ void enqueue_junction(tp_context *c, bool prim = false) {
 void enqueue_avg(tp_context *c, bool prim = false) {
   StageArgs a = base_args(c);
   run_faces(c, c->L.acap, FK_AVG_CAP, a, K_GCBC);
-  run_faces(c, c->L.acap, FK_COPY, a, K_GCBC);
   a.opt = prim ? 1 : 0;
-  for (int d = 0; d < 3; d++) run_faces(c, c->L.aapply[d], FK_AVG_APPLY, a, K_GCBC);
+  run_faces(c, c->L.acap, FK_AVG_APPLY, a, K_GCBC);
 }
 
 // one stage, src/Main3D.f90:567-958: the stresses and heat fluxes stay in
@@ -1401,7 +1399,7 @@ int build_case(HostCase &h) {
 
 // launch tables over the global blocks gs (sorted by case)
 int make_lists(tp_context *c, const std::vector<int> &gs, Mem &m, ListSet &L) {
-  std::vector<Work> pts, sp, fo, lw[3], ex, gp, ga[3], gc, wl, ac, aa[3], nm, sf;
+  std::vector<Work> pts, sp, fo, lw[3], ex, gp, ga[3], wl, ac, nm, sf;
   L.wr.assign(c->linked.size() + 1, 0);
   L.wwr.assign(c->linked.size() + 1, 0);
   int slot = -1;
@@ -1440,9 +1438,8 @@ int make_lists(tp_context *c, const std::vector<int> &gs, Mem &m, ListSet &L) {
         const bool wall = np == 20 || np == 25;
         if (b.ndf[d][s]) add(ex);
         if (gc_face) { add(gp); add(ga[d]); }
-        if (np == 30 || (gcic && wall)) add(gc);
         if (wall) add(wl);
-        if (np == 30 || np == 35 || np == 45 || (gcic && wall)) { add(ac); add(aa[d]); }
+        if (np == 30 || np == 35 || np == 45 || (gcic && wall)) add(ac);
         add(nm);
       }
   }
@@ -1458,14 +1455,12 @@ int make_lists(tp_context *c, const std::vector<int> &gs, Mem &m, ListSet &L) {
   if ((rc = upload_list(m, L.force, fo))) return rc;
   if ((rc = upload_list(m, L.exch, ex))) return rc;
   if ((rc = upload_list(m, L.gprep, gp))) return rc;
-  if ((rc = upload_list(m, L.gcopy, gc))) return rc;
   if ((rc = upload_list(m, L.wall, wl))) return rc;
   if ((rc = upload_list(m, L.acap, ac))) return rc;
   if ((rc = upload_list(m, L.normals, nm))) return rc;
   for (int d = 0; d < 3; d++) {
     if ((rc = upload_list(m, L.lines[d], lw[d]))) return rc;
     if ((rc = upload_list(m, L.gapply[d], ga[d]))) return rc;
-    if ((rc = upload_list(m, L.aapply[d], aa[d]))) return rc;
   }
   return 0;
 }

@@ -343,9 +343,9 @@ __device__ inline const double *stage_q(const StageArgs &a, const Block &b) { re
 // face kernels' points).  1/rho (de(:,1)) and the viscosity (ss(:,1)) are
 // read only by the time-step limit, which follows the primitives pass of a
 // step's first stage; the flux pass forms the viscosity again from q.
-__device__ inline void put_primitives(const Block &b, const CaseCoef &c, const Phys &ph, int l) {
+__device__ inline void put_primitives(const Block &b, const CaseCoef &c, const Phys &ph, int l, const double q[5]) {
   const int N = b.N;
-  const Prim r = primitives(c, ph, b.qa[l], b.qa[N + l], b.qa[2 * N + l], b.qa[3 * N + l], b.qa[4 * N + l]);
+  const Prim r = primitives(c, ph, q[0], q[1], q[2], q[3], q[4]);
   b.de[N + l] = r.d2; b.de[2 * N + l] = r.d3; b.de[3 * N + l] = r.d4; b.de[4 * N + l] = r.d5;
   b.p[l] = r.p;
 }
@@ -837,16 +837,19 @@ __global__ void __launch_bounds__(256) k_gcbc_prep(StageArgs a) {
   }
 }
 
-// ---- face copy from the neighbour: drvb(:,:,ip) <- drva(:,:,1-ip) of ncd
-// (GCIC exchange Main3D.f90:799-813 and interface averaging :915-925) ----
-__global__ void __launch_bounds__(256) k_face_copy(StageArgs a) {
-  const Work w = a.work[xcd_item(blockIdx.x, gridDim.x)];
-  const Block &b = a.blocks[w.blk];
-  const int d = w.d & 0xff, ip = w.d >> 8, F = b.F[d];
-  int jk;
-  if (!face_point(b, w, d, jk)) return;
-  const Block &s = a.blocks[b.ncd[d][ip]];
-  for (int c = 0; c < 5; c++) b.drvb[d][(ip * 5 + c) * F + jk] = s.drva[d][((1 - ip) * 5 + c) * F + jk];
+// ---- the neighbour's value of an interface face point: drvb(:,:,ip) <-
+// drva(:,:,1-ip) of ncd (GCIC exchange Main3D.f90:799-813 and interface
+// averaging :915-925) ----
+// The kernels that use it read the neighbour's drva themselves (nothing they
+// run beside writes it) and leave it in drvb: a launch between the two that
+// only copied face arrays took 3.5-10 us, twice a stage.
+__device__ inline void face_partner(const Block *blocks, const Block &b, int d, int ip, int jk, double o[5]) {
+  const Block &s = blocks[b.ncd[d][ip]];
+  const int F = b.F[d];
+#pragma unroll
+  for (int c = 0; c < 5; c++) o[c] = s.drva[d][((1 - ip) * 5 + c) * F + jk];
+#pragma unroll
+  for (int c = 0; c < 5; c++) b.drvb[d][(ip * 5 + c) * F + jk] = o[c];
 }
 
 // number of characteristic faces whose band (face point + MBCI inward) holds
@@ -906,7 +909,13 @@ __global__ void __launch_bounds__(256) k_gcbc_apply(StageArgs a) {
     Elem e;
     eleme(q, pl, cm, sc + S_UMF1, e);
     const double *drva = b.drva[d], *drvb = b.drvb[d];
-    for (int v = 0; v < 5; v++) { cha[v] = drva[(ip * 5 + v) * F + jk]; dha[v] = drvb[(ip * 5 + v) * F + jk]; }
+    for (int v = 0; v < 5; v++) cha[v] = drva[(ip * 5 + v) * F + jk];
+    // the faces that exchange: interfaces, and with GCIC the walls
+    if (np == 30 || (c.nextgcic == 1 && (np == 20 || np == 25))) {
+      face_partner(a.blocks, b, d, ip, jk, dha);
+    } else {
+      for (int v = 0; v < 5; v++) dha[v] = drvb[(ip * 5 + v) * F + jk];
+    }
     double vv = e.vn + e.vs;
     if (np == 10) {
       if (ra0 * (vv + e.ao) > 0.0) cha[3] = 0.0;
@@ -964,7 +973,8 @@ __global__ void __launch_bounds__(256) k_gcbc_apply(StageArgs a) {
   // band point's weight is formed once for its five fields: with one element
   // per loop turn, index divisions and all, the read-modify-write chain of 20
   // memory latencies was the kernel (19.3 us a launch for 2 k face points in 12
-  // workgroups, now 7.8; 60 us for 233 k, now 45).
+  // workgroups, now 7.8, or 8.9 with the partner faces' copy to drvb; 60 us for
+  // 233 k, now 66 with that copy, which took 10 in a launch of its own).
   constexpr int NB = MBCI + 1, NG = 4;
   static_assert(NB == 4, "a thread's band point is its low two bits");
   const int ii = threadIdx.x & (NB - 1);
@@ -1049,8 +1059,9 @@ __global__ void __launch_bounds__(256) k_wall(StageArgs a) {
   double fctr = (1.0 - ra3) * qa[l];
   for (int v = 0; v < 3; v++) qa[(1 + v) * N + l] = ra3 * qa[(1 + v) * N + l] - fctr * umf[v];
   double q1 = qa[l], q2 = qa[N + l], q3 = qa[2 * N + l], q4 = qa[3 * N + l];
-  qa[4 * N + l] = rp * qa[4 * N + l] + ra2 * (ra0 * q1 + 0.5 * (q2 * q2 + q3 * q3 + q4 * q4) / q1);
-  if (a.opt) put_primitives(b, c, ph, l);   // the next stage's primitives, formed in the update
+  const double q[5] = {q1, q2, q3, q4, rp * qa[4 * N + l] + ra2 * (ra0 * q1 + 0.5 * (q2 * q2 + q3 * q3 + q4 * q4) / q1)};
+  qa[4 * N + l] = q[4];
+  if (a.opt) put_primitives(b, c, ph, l, q);   // the next stage's primitives, formed in the update
 }
 
 // ---- junction averaging, SingleTurbulence3D.f90:378-443 ----
@@ -1080,7 +1091,7 @@ __global__ void k_junction(const Block *blocks, const CaseCoef *coef, const int 
   for (int q = 0; q < 4; q++) {
     const Block &b = blocks[J[q * 3]];
     for (int m = 0; m < 5; m++) b.qa[(size_t)m * b.N + lq[q]] = r[m];
-    if (prim) put_primitives(b, coef[b.cs], phys(), lq[q]);
+    if (prim) put_primitives(b, coef[b.cs], phys(), lq[q], r);
   }
 }
 
@@ -1124,6 +1135,19 @@ __device__ inline double avg_count(const Block &b, const CaseCoef &c, int x, int
   return cnt + self_inc;
 }
 
+// whether the interface averaging works on face (d, ip) of block b
+__device__ inline bool avg_face(const Block &b, const CaseCoef &c, int d, int ip) {
+  const int np = b.nbc[d][ip];
+  return avg_code(np) || (c.nextgcic == 1 && (np == 20 || np == 25));
+}
+
+// The reference averages face by face: xi, eta, zeta (the two faces of a
+// direction share no point, lines having >= 7 points).  Only a point's own
+// running average depends on that order, so one launch does every face: the
+// thread of the point's first averaged face carries it through the others in
+// turn, the threads of the others leave it alone.  (Three launches took 16-17 us a
+// stage at 28 k and 208 k points, one, with the copy to drvb, 7-8 us; 54 and
+// 40 us at 20 M points.)
 __global__ void __launch_bounds__(256) k_avg_apply(StageArgs a) {
   const Work w = a.work[xcd_item(blockIdx.x, gridDim.x)];
   const Block &b = a.blocks[w.blk];
@@ -1131,36 +1155,43 @@ __global__ void __launch_bounds__(256) k_avg_apply(StageArgs a) {
   const int N = b.N, d = w.d & 0xff, ip = w.d >> 8, F = b.F[d];
   int jk;
   if (!face_point(b, w, d, jk)) return;
-  const int np = b.nbc[d][ip];
   int j, k;
   face_jk(b, d, jk, j, k);
-  int l = indx3(b, ip * (b.L[d] - 1), j, k, d);
+  const int l = indx3(b, ip * (b.L[d] - 1), j, k, d);
+  // the point's captured state: contiguous in the face array, while qa holds
+  // a xi face's points a row apart
+  double q[5], o[5];
+  for (int v = 0; v < 5; v++) q[v] = b.drva[d][(ip * 5 + v) * F + jk];
+  face_partner(a.blocks, b, d, ip, jk, o);
   int x, y, z;
   point_ijk(b, l, x, y, z);
-  // a face of the same direction at the other end cannot hold this point
-  // (lines have >= 7 points), so only earlier directions contribute
-  double *qa = b.qa;
-  const double *drvb = b.drvb[d];
-  // the point's state: on xi faces (the first direction) the value captured
-  // for this face, from one face array each instead of a row per point (no
-  // earlier direction has changed it); later directions read qa, which an
-  // earlier face of the point may have averaged
-  double q[5];
-  for (int v = 0; v < 5; v++) q[v] = d == 0 ? b.drva[0][(ip * 5 + v) * F + jk] : qa[(size_t)v * N + l];
-  if (avg_code(np)) {
-    double r1 = avg_count(b, c, x, y, z, d, 1.0);
-    double r2 = 1.0 / r1;
-    for (int v = 0; v < 5; v++)
-      qa[(size_t)v * N + l] = r2 * ((r1 - 1.0) * q[v] + drvb[(ip * 5 + v) * F + jk]);
-  } else {
-    double rp = b.rpex[b.wall_off[d][ip] + jk];
-    double ra1 = 1.0 - rp;
-    double r1 = avg_count(b, c, x, y, z, d, rp);
-    double r2 = 1.0 / r1;
-    for (int v = 0; v < 5; v++)
-      qa[(size_t)v * N + l] = rp * r2 * ((r1 - 1.0) * q[v] + drvb[(ip * 5 + v) * F + jk]) + ra1 * q[v];
+  const int idx[3] = {x, y, z};
+  for (int e = 0; e < d; e++) {
+    if (idx[e] == 0 && avg_face(b, c, e, 0)) return;
+    if (idx[e] == b.L[e] - 1 && avg_face(b, c, e, 1)) return;
   }
-  if (a.opt) put_primitives(b, c, phys(), l);   // the next stage's primitives, formed in the update
+  for (int e = d; e < 3; e++) {
+    int se = ip, je = jk;
+    if (e > d) {
+      if (idx[e] == 0 && avg_face(b, c, e, 0)) se = 0;
+      else if (idx[e] == b.L[e] - 1 && avg_face(b, c, e, 1)) se = 1;
+      else continue;
+      je = e == 1 ? x * b.nz + z : y * b.nx + x;
+      const Block &s = a.blocks[b.ncd[e][se]];
+      for (int v = 0; v < 5; v++) o[v] = s.drva[e][((1 - se) * 5 + v) * b.F[e] + je];
+    }
+    if (avg_code(b.nbc[e][se])) {
+      const double r1 = avg_count(b, c, x, y, z, e, 1.0), r2 = 1.0 / r1;
+      for (int v = 0; v < 5; v++) q[v] = r2 * ((r1 - 1.0) * q[v] + o[v]);
+    } else {
+      const double rp = b.rpex[b.wall_off[e][se] + je], ra1 = 1.0 - rp;
+      const double r1 = avg_count(b, c, x, y, z, e, rp), r2 = 1.0 / r1;
+      for (int v = 0; v < 5; v++) q[v] = rp * r2 * ((r1 - 1.0) * q[v] + o[v]) + ra1 * q[v];
+    }
+  }
+  for (int v = 0; v < 5; v++) b.qa[(size_t)v * N + l] = q[v];
+  // the next stage's primitives, formed in the update
+  if (a.opt) put_primitives(b, c, phys(), l, q);
 }
 
 // ---- copies ----
@@ -1363,7 +1394,6 @@ void launch_point(int which, int nwg, hipStream_t st, const StageArgs &a) {
 void launch_face(int which, int nwg, hipStream_t st, const StageArgs &a) {
   switch (which) {
     case 0: LAUNCH(k_gcbc_prep, nwg, 256, st, a); break;
-    case 1: LAUNCH(k_face_copy, nwg, 256, st, a); break;
     case 2: LAUNCH(k_gcbc_apply<false>, nwg, 256, st, a); break;
     case 3: LAUNCH(k_wall, nwg, 256, st, a); break;
     case 4: LAUNCH(k_avg_capture, nwg, 256, st, a); break;
