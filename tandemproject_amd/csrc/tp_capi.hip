@@ -507,6 +507,8 @@ struct tp_context {
   size_t lds[3] = {0, 0, 0};
   bool exact_lines = false;        // sequential one-lane-per-line sweeps
   bool keep_stress = false;        // tv written at every point of every stage
+  int phase = 0;                   // scalar row of kernels enqueued now: 0, inside a whole time
+                                   // step k from stage k's update on (set by enqueue_step only)
   bool qin = false;                // kernels enqueued now read the stage's state from qo
                                    // (StageArgs::qin): set by enqueue_step only
   int col_fixed = 0;               // requested chunks per line (0: chosen per direction)
@@ -638,7 +640,7 @@ StageArgs base_args(tp_context *c) {
   std::memset(&a, 0, sizeof(a));
   a.blocks = c->d_blocks;
   a.coef = c->d_coef;
-  a.sc = c->d_sc;
+  a.sc = c->d_sc + (size_t)c->phase * c->linked.size() * S_STRIDE;
   a.part = c->d_part;
   a.wpart = c->d_wpart;
   a.qin = c->qin ? 1 : 0;
@@ -910,9 +912,8 @@ void enqueue_filter_step(tp_context *c, bool lean = false) {
 // viscosity only on the steps whose time-step limit reads them
 void enqueue_begin(tp_context *c, int nk, bool prim_ready = false, bool lean = false) {
   const int ncase = (int)c->linked.size();
-  // (with prim_ready the previous stage's k_sc_rk left this stage's start
-  // scalars too)
-  if (!prim_ready) launch_sc_stage(c->d_coef, c->d_sc, ncase, nk, c->stream);
+  // (inside a whole time step k_sc_dt forms the scalars of every stage)
+  if (!prim_ready) launch_sc_stage(c->d_coef, c->d_sc, ncase, nk, lean ? 1 : 0, c->stream);
   StageArgs a = base_args(c);
   a.nk = nk;
   a.opt = lean ? 1 : 0;
@@ -920,7 +921,7 @@ void enqueue_begin(tp_context *c, int nk, bool prim_ready = false, bool lean = f
   a.opt = 0;
   if (nk == 1) {
     run_points(c, PK_DTRED, a, K_POINT, 0.0);
-    launch_sc_dt(c->d_coef, c->d_sc, c->d_part, c->d_wr, ncase, 1, c->stream);
+    launch_sc_dt(c->d_coef, c->d_sc, c->d_part, c->d_wr, ncase, lean ? 1 : 0, c->stream);
   }
 }
 
@@ -987,8 +988,9 @@ void enqueue_gcbc(tp_context *c) {
 // and averaging passes after it form them again where they change the state,
 // so that the next stage starts without the primitives pass and its read of
 // qa (the residual in de is read first)
-void enqueue_rk(tp_context *c, int nk, bool prim = false) {
-  launch_sc_rk(c->d_coef, c->d_sc, (int)c->linked.size(), nk, prim ? 1 : 0, c->stream);
+void enqueue_rk(tp_context *c, int nk, bool prim = false, bool lean = false) {
+  if (lean) c->phase = nk;
+  else launch_sc_rk(c->d_coef, c->d_sc, (int)c->linked.size(), nk, c->stream);
   StageArgs a = base_args(c);
   a.nk = nk;
   if (prim) run_points(c, PK_RK_PRIM, a, K_RK, 168.0);
@@ -1036,7 +1038,7 @@ void enqueue_stage(tp_context *c, int nk, bool prim_ready = false, bool prim_nex
   enqueue_sponge(c);
   enqueue_gcbc(c);
   c->qin = false;   // the update reads qo and writes qa in any case
-  enqueue_rk(c, nk, prim_next);
+  enqueue_rk(c, nk, prim_next, lean);
   enqueue_wall(c, prim_next);
   enqueue_junction(c, prim_next);
   enqueue_avg(c, prim_next);
@@ -1050,7 +1052,8 @@ void enqueue_step(tp_context *c) {
   c->qin = true;    // until the first stage's update
   for (int nk = 1; nk <= c->nkrk; nk++) enqueue_stage(c, nk, nk > 1, nk < c->nkrk, true);
   c->qin = false;
-  launch_sc_end(c->d_sc, (int)c->linked.size(), nullptr, c->stream);
+  c->phase = 0;
+  launch_sc_end(c->d_coef, c->d_sc, (int)c->linked.size(), c->stream);
 }
 
 int check_ready(tp_context *c) {
@@ -1538,6 +1541,7 @@ int link(tp_context *c) {
   if ((rc = make_groups(c, gs, c->lmem, c->L))) return rc;
   if ((rc = upload_vec(c->link, &c->d_blocks, c->blocks))) return rc;
   if ((rc = upload_vec(c->link, &c->d_coef, coefs))) return rc;
+  sc.resize(sc.size() * (size_t)(c->nkrk + 1), 0.0);   // row 0, and a row per stage (k_sc_dt)
   if ((rc = upload_vec(c->link, &c->d_sc, sc))) return rc;
   std::vector<double> part(2 * std::max(c->L.points.n, 1), 0.0);
   if ((rc = upload_vec(c->link, &c->d_part, part))) return rc;

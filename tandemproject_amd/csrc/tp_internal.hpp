@@ -258,7 +258,7 @@ struct StageArgs {
   const Block *blocks;
   const Work *work;
   const CaseCoef *coef;
-  double *sc;        // [ncase][S_STRIDE]
+  double *sc;        // [ncase][S_STRIDE]: the current phase's row
   double *part;      // reduction partials [nwork][2]
   double *wpart;     // wall-force partials [nwallwork][4]
   int nk, m, d, opt; // stage number, field, direction, option (k_flux_all: write tv everywhere;
@@ -297,12 +297,13 @@ void launch_filter(int d, int nwg, int nf, size_t lds, hipStream_t st, const Lin
 void launch_exchange(int nwg, int nf, hipStream_t st, const ExchArgs &a);
 void launch_point(int which, int nwg, hipStream_t st, const StageArgs &a);
 void launch_face(int which, int nwg, hipStream_t st, const StageArgs &a);
-void launch_sc_stage(const CaseCoef *coef, double *sc, int ncase, int nk, hipStream_t st);
+void launch_sc_stage(const CaseCoef *coef, double *sc, int ncase, int nk, int limit, hipStream_t st);
+// ahead (inside a whole time step): also the scalars of every stage's start
+// and update, rows of sc
 void launch_sc_dt(const CaseCoef *coef, double *sc, const double *part, const int *wr, int ncase,
-                  int reduced, hipStream_t st);
-// next: also the next stage's start scalars (inside a whole time step)
-void launch_sc_rk(const CaseCoef *coef, double *sc, int ncase, int nk, int next, hipStream_t st);
-void launch_sc_end(double *sc, int ncase, const int *active, hipStream_t st);
+                  int ahead, hipStream_t st);
+void launch_sc_rk(const CaseCoef *coef, double *sc, int ncase, int nk, hipStream_t st);
+void launch_sc_end(const CaseCoef *coef, double *sc, int ncase, hipStream_t st);
 void launch_junction(const Block *blocks, const CaseCoef *coef, const int *jct, const int *jvel, int njct, int maxk,
                      int prim, hipStream_t st);
 void launch_surf_reduce(const CaseCoef *coef, double *sc, const double *wpart, const int *wwr, int ncase,

@@ -214,11 +214,14 @@ __device__ void inflow_weights(const CaseCoef &c, double *s) {
   s[S_LAGON] = 1.0;
 }
 
-__global__ void k_sc_stage(const CaseCoef *coef, double *sc, int ncase, int nk) {
+// limit (inside a whole time step, where k_sc_dt forms the scalars of every
+// stage): only on the steps whose time-step limit reads the frame velocity
+__global__ void k_sc_stage(const CaseCoef *coef, double *sc, int ncase, int nk, int limit) {
   int cs = blockIdx.x * blockDim.x + threadIdx.x;
   if (cs >= ncase) return;
   const CaseCoef &c = coef[cs];
   double *s = sc + cs * S_STRIDE;
+  if (limit && (int)s[S_N] % 10 != 1) return;
   int nkrk = c.nkrk;
   double dt = s[S_DT];
   int f1 = nk - 2 > 0 ? (nk - 2 < 1 ? nk - 2 : 1) : 0;
@@ -231,15 +234,23 @@ __global__ void k_sc_stage(const CaseCoef *coef, double *sc, int ncase, int nk) 
 
 // time step size: Main3D.f90:587-610 (maxima reduced from the partials of the
 // blocks of each case; wr[cs], wr[cs+1] bound its work items)
+// ahead (inside a whole time step): with the step size known, every scalar
+// that the stages' starts and updates form (k_sc_stage, k_sc_rk) is too, so
+// they are formed here side by side, one thread per phase: row 0 of sc the
+// first stage's start, row k >= 1 stage k's update and stage k+1's start.  A
+// scalar kernel before every update cost 6.7 us a stage at 28 k points and
+// 14.4 at 20 M, all of it the latency of one thread's double-double sines;
+// this one takes 10.6 and 34 us instead of 5.3 and 18.6, and the first
+// stage's own (6.2, 15.5) returns at once on nine steps of ten.
 __global__ void k_sc_dt(const CaseCoef *coef, double *sc, const double *part, const int *wr,
-                        int ncase, int reduced) {
+                        int ncase, int ahead) {
   int cs = blockIdx.x;
   if (cs >= ncase) return;
   __shared__ double mi[256], mv[256];
   double fi = -INFINITY, fv = -INFINITY;
   double *s = sc + cs * S_STRIDE;
   int n = (int)s[S_N];
-  bool need = reduced && (n % 10 == 1) && coef[cs].dto < 0.0;
+  bool need = (n % 10 == 1) && coef[cs].dto < 0.0;
   if (need) {
     for (int q = wr[cs] + threadIdx.x; q < wr[cs + 1]; q += blockDim.x) {
       fi = fmax(fi, part[2 * q]);
@@ -271,14 +282,28 @@ __global__ void k_sc_dt(const CaseCoef *coef, double *sc, const double *part, co
     double sn = cr_sin(0.05 * PI_D * (double)(n - (int)s[S_NDT]));
     s[S_DT] = s[S_DTS] + (s[S_DTE] - s[S_DTS]) * (sn * sn);
   }
+  if (!ahead) return;
+  __syncthreads();
+  // the frame arguments of a stage's update are those of the next stage's
+  // start: the same time, the same step
+  const CaseCoef &c = coef[cs];
+  const int nkrk = c.nkrk;
+  for (int t = threadIdx.x; t <= nkrk; t += blockDim.x) {
+    double *r = sc + ((size_t)t * ncase + cs) * S_STRIDE;
+    double dtko = 0.0, dtk = 0.0;
+    if (t > 0) {
+      for (int q = 0; q < S_NSCALAR; q++) r[q] = s[q];
+      const double dt = s[S_DT];
+      dtko = dt * (double)(t - 1 < 1 ? t - 1 : 1) / (nkrk - t + 2);
+      dtk = dt / (nkrk - t + 1);
+    }
+    movef_dev(c, r, dtko, dtk);
+    if (c.inflow && t < nkrk) inflow_weights(c, r);
+  }
 }
 
-// before the RK update: Main3D.f90:873-874.  Its frame arguments (dtko, dtk)
-// are those of the next stage's start (k_sc_stage(nk + 1): the same time,
-// the same step), so with next set (inside a whole time step) it also forms
-// the next stage's inflow weights and that stage needs no k_sc_stage; this
-// stage's sponge, their only reader, has run.
-__global__ void k_sc_rk(const CaseCoef *coef, double *sc, int ncase, int nk, int next) {
+// before the RK update: Main3D.f90:873-874
+__global__ void k_sc_rk(const CaseCoef *coef, double *sc, int ncase, int nk) {
   int cs = blockIdx.x * blockDim.x + threadIdx.x;
   if (cs >= ncase) return;
   const CaseCoef &c = coef[cs];
@@ -288,14 +313,19 @@ __global__ void k_sc_rk(const CaseCoef *coef, double *sc, int ncase, int nk, int
   double dtko = dt * (double)f2 / (c.nkrk - nk + 2);
   double dtk = dt / (c.nkrk - nk + 1);
   movef_dev(c, s, dtko, dtk);
-  if (next && c.inflow) inflow_weights(c, s);
 }
 
-// end of step: Main3D.f90:964-965
-__global__ void k_sc_end(double *sc, int ncase, const int *active) {
+// end of a whole step: Main3D.f90:964-965, and the frame scalars as the last
+// update left them, the inflow weights as the last stage's start did
+__global__ void k_sc_end(const CaseCoef *coef, double *sc, int ncase) {
   int cs = blockIdx.x * blockDim.x + threadIdx.x;
-  if (cs >= ncase || (active && !active[cs])) return;
+  if (cs >= ncase) return;
   double *s = sc + cs * S_STRIDE;
+  const int nkrk = coef[cs].nkrk;
+  const double *last = s + (size_t)nkrk * ncase * S_STRIDE, *start = last - (size_t)ncase * S_STRIDE;
+  for (int q = S_UMF1; q <= S_AOA; q++) s[q] = last[q];
+  if (nkrk > 1 && coef[cs].inflow)
+    for (int q = S_LAGW; q <= S_LAGON; q++) s[q] = start[q];
   s[S_N] = s[S_N] + 1;
   s[S_TIMO] = s[S_TIMO] + s[S_DT];
 }
@@ -1408,18 +1438,18 @@ void launch_surf_reduce(const CaseCoef *coef, double *sc, const double *wpart, c
                         hipStream_t st) {
   hipLaunchKernelGGL(k_surf_reduce, dim3(ncase), dim3(256), 0, st, coef, sc, wpart, wwr, ncase);
 }
-void launch_sc_stage(const CaseCoef *coef, double *sc, int ncase, int nk, hipStream_t st) {
-  hipLaunchKernelGGL(k_sc_stage, dim3((ncase + 63) / 64), dim3(64), 0, st, coef, sc, ncase, nk);
+void launch_sc_stage(const CaseCoef *coef, double *sc, int ncase, int nk, int limit, hipStream_t st) {
+  hipLaunchKernelGGL(k_sc_stage, dim3((ncase + 63) / 64), dim3(64), 0, st, coef, sc, ncase, nk, limit);
 }
-void launch_sc_dt(const CaseCoef *coef, double *sc, const double *part, const int *wr, int ncase, int reduced,
+void launch_sc_dt(const CaseCoef *coef, double *sc, const double *part, const int *wr, int ncase, int ahead,
                   hipStream_t st) {
-  hipLaunchKernelGGL(k_sc_dt, dim3(ncase), dim3(256), 0, st, coef, sc, part, wr, ncase, reduced);
+  hipLaunchKernelGGL(k_sc_dt, dim3(ncase), dim3(256), 0, st, coef, sc, part, wr, ncase, ahead);
 }
-void launch_sc_rk(const CaseCoef *coef, double *sc, int ncase, int nk, int next, hipStream_t st) {
-  hipLaunchKernelGGL(k_sc_rk, dim3((ncase + 63) / 64), dim3(64), 0, st, coef, sc, ncase, nk, next);
+void launch_sc_rk(const CaseCoef *coef, double *sc, int ncase, int nk, hipStream_t st) {
+  hipLaunchKernelGGL(k_sc_rk, dim3((ncase + 63) / 64), dim3(64), 0, st, coef, sc, ncase, nk);
 }
-void launch_sc_end(double *sc, int ncase, const int *active, hipStream_t st) {
-  hipLaunchKernelGGL(k_sc_end, dim3((ncase + 63) / 64), dim3(64), 0, st, sc, ncase, active);
+void launch_sc_end(const CaseCoef *coef, double *sc, int ncase, hipStream_t st) {
+  hipLaunchKernelGGL(k_sc_end, dim3((ncase + 63) / 64), dim3(64), 0, st, coef, sc, ncase);
 }
 void launch_junction(const Block *blocks, const CaseCoef *coef, const int *jct, const int *jvel, int njct, int maxk,
                      int prim, hipStream_t st) {
