@@ -983,26 +983,25 @@ void enqueue_gcbc(tp_context *c) {
 }
 
 // frame velocity for the update and the RK update, src/Main3D.f90:873-881
+// wall: with the wall conditions (src/Main3D.f90:884-895), as a whole stage
+// has them right after the update
 // prim: the update also leaves the primitives the next stage reads
-// (de(:,2:5) and p of the new state, k_primitives' arithmetic), and the wall, junction
+// (de(:,2:5) and p of the new state, k_primitives' arithmetic), and the junction
 // and averaging passes after it form them again where they change the state,
 // so that the next stage starts without the primitives pass and its read of
 // qa (the residual in de is read first)
-void enqueue_rk(tp_context *c, int nk, bool prim = false, bool lean = false) {
+void enqueue_rk(tp_context *c, int nk, bool wall, bool prim = false, bool lean = false) {
   if (lean) c->phase = nk;
   else launch_sc_rk(c->d_coef, c->d_sc, (int)c->linked.size(), nk, c->stream);
   StageArgs a = base_args(c);
   a.nk = nk;
+  a.opt = wall ? 1 : 0;
   if (prim) run_points(c, PK_RK_PRIM, a, K_RK, 168.0);
   else run_points(c, PK_RK, a, K_RK, 128.0);
 }
 
 // wall temperature and velocity, src/Main3D.f90:884-895
-void enqueue_wall(tp_context *c, bool prim = false) {
-  StageArgs a = base_args(c);
-  a.opt = prim ? 1 : 0;
-  run_faces(c, c->L.wall, FK_WALL, a, K_GCBC);
-}
+void enqueue_wall(tp_context *c) { run_faces(c, c->L.wall, FK_WALL, base_args(c), K_GCBC); }
 
 // corner junctions, src/SingleTurbulence3D.f90:378-443
 void enqueue_junction(tp_context *c, bool prim = false) {
@@ -1038,8 +1037,7 @@ void enqueue_stage(tp_context *c, int nk, bool prim_ready = false, bool prim_nex
   enqueue_sponge(c);
   enqueue_gcbc(c);
   c->qin = false;   // the update reads qo and writes qa in any case
-  enqueue_rk(c, nk, prim_next, lean);
-  enqueue_wall(c, prim_next);
+  enqueue_rk(c, nk, true, prim_next, lean);
   enqueue_junction(c, prim_next);
   enqueue_avg(c, prim_next);
 }
@@ -2330,7 +2328,7 @@ int32_t tp_gcbc(tp_context *c) {
 
 int32_t tp_rk_update(tp_context *c, int32_t nk) {
   if (int rc = stage_ok(c, nk)) return rc;
-  if (!c->linked.empty()) enqueue_rk(c, nk);
+  if (!c->linked.empty()) enqueue_rk(c, nk, false);
   return launched();
 }
 

@@ -262,7 +262,8 @@ struct StageArgs {
   double *part;      // reduction partials [nwork][2]
   double *wpart;     // wall-force partials [nwallwork][4]
   int nk, m, d, opt; // stage number, field, direction, option (k_flux_all: write tv everywhere;
-                     // k_wall, k_avg_apply: form the primitives of the points they change)
+                     // k_rk: apply the wall conditions too; k_avg_apply: form the primitives
+                     // of the points it changes)
   int arr, col;      // generic field selector
   int o0, o1, o2;    // tv slots for gradient combination (-1..-3 = ss columns)
   int qin;           // 1: the stage's state is in qo, not qa, until its update (the

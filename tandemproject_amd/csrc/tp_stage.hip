@@ -1038,24 +1038,56 @@ __global__ void __launch_bounds__(256) k_gcbc_apply(StageArgs a) {
   }
 }
 
+// ---- wall temperature and velocity of one wall-face point's state q,
+// Main3D.f90:886-895 (rp: the point's wall-slot flag) ----
+__device__ inline void wall_state(const CaseCoef &c, const Phys &ph, int np, double rp, const double *umf,
+                                  double q[5]) {
+  const double ra0 = ph.ham * ph.hamm1 * c.wtemp;
+  const double ra1 = (double)((np - 20) / 5);
+  const double ra2 = 1.0 - rp, ra3 = 1.0 - ra1 * ra2;
+  const double fctr = (1.0 - ra3) * q[0];
+  for (int v = 0; v < 3; v++) q[1 + v] = ra3 * q[1 + v] - fctr * umf[v];
+  q[4] = rp * q[4] + ra2 * (ra0 * q[0] + 0.5 * (q[1] * q[1] + q[2] * q[2] + q[3] * q[3]) / q[0]);
+}
+
+__device__ inline bool wall_code(int np) { return np == 20 || np == 25; }
+
 // ---- RK update, Main3D.f90:876-881 ----
 // PRIM: also the next stage's primitives of the updated state (k_primitives'
 // arithmetic on the same values) that the stage reads, u, v, w, T into
-// de(:,2:5) and p, once the residual is read; the wall, junction and
-// averaging passes that follow form them again at the points they change
+// de(:,2:5) and p, once the residual is read; the junction and averaging
+// passes that follow form them again at the points they change
+// opt: also the wall conditions at the points of wall faces, which need
+// nothing but the point's own state (a launch of their own took 4.4 us a stage at 28 k
+// points and 6.0 at 20 M; the steps are 2.6 % shorter at 28 k and 1.2 % at 1 M
+// points, the same within 0.2 % at 20 M)
 template <bool PRIM>
 __global__ void __launch_bounds__(256) k_rk(StageArgs a) {
   WORK_POINTS
-  const double dtk = a.sc[b.cs * S_STRIDE + S_DTK];
+  const double *sc = a.sc + b.cs * S_STRIDE;
+  const double dtk = sc[S_DTK];
   const CaseCoef &c = a.coef[b.cs];
   const Phys ph = phys();
+  bool walls = false;
+  if (a.opt)
+    for (int d = 0; d < 3; d++) walls = walls || wall_code(b.nbc[d][0]) || wall_code(b.nbc[d][1]);
   for (int l = w.a + threadIdx.x; l < w.a + w.n; l += blockDim.x) {
     double r1 = dtk * ld_stream(&b.yaco[l]);
     double q[5];
-    for (int v = 0; v < 5; v++) {
+    for (int v = 0; v < 5; v++)
       q[v] = ld_stream(&b.qo[(size_t)v * N + l]) - r1 * ld_stream(&b.de[(size_t)v * N + l]);
-      st_stream(&b.qa[(size_t)v * N + l], q[v]);
+    if (walls) {
+      int x, y, z;
+      point_ijk(b, l, x, y, z);
+      const int idx[3] = {x, y, z};
+      for (int d = 0; d < 3; d++) {
+        const int s = idx[d] == 0 ? 0 : 1;
+        if ((idx[d] != 0 && idx[d] != b.L[d] - 1) || !wall_code(b.nbc[d][s])) continue;
+        const int jk = d == 0 ? z * b.ny + y : d == 1 ? x * b.nz + z : y * b.nx + x;
+        wall_state(c, ph, b.nbc[d][s], b.rpex[b.wall_off[d][s] + jk], sc + S_UMF1, q);
+      }
     }
+    for (int v = 0; v < 5; v++) st_stream(&b.qa[(size_t)v * N + l], q[v]);
     if (PRIM) {
       const Prim r = primitives(c, ph, q[0], q[1], q[2], q[3], q[4]);
       st_stream(&b.de[N + l], r.d2);
@@ -1067,31 +1099,20 @@ __global__ void __launch_bounds__(256) k_rk(StageArgs a) {
   }
 }
 
-// ---- wall temperature and velocity, Main3D.f90:886-895 ----
+// ---- the wall conditions alone (the wall drop-in) ----
 __global__ void __launch_bounds__(256) k_wall(StageArgs a) {
   const Work w = a.work[xcd_item(blockIdx.x, gridDim.x)];
   const Block &b = a.blocks[w.blk];
-  const CaseCoef &c = a.coef[b.cs];
-  const Phys ph = phys();
   const int N = b.N, d = w.d & 0xff, ip = w.d >> 8;
   int jk;
   if (!face_point(b, w, d, jk)) return;
-  const int np = b.nbc[d][ip];
-  const double *umf = a.sc + b.cs * S_STRIDE + S_UMF1;
   int j, k;
   face_jk(b, d, jk, j, k);
-  int l = indx3(b, ip * (b.L[d] - 1), j, k, d);
-  double ra0 = ph.ham * ph.hamm1 * c.wtemp;
-  double ra1 = (double)((np - 20) / 5);
-  double rp = b.rpex[b.wall_off[d][ip] + jk];
-  double ra2 = 1.0 - rp, ra3 = 1.0 - ra1 * ra2;
-  double *qa = b.qa;
-  double fctr = (1.0 - ra3) * qa[l];
-  for (int v = 0; v < 3; v++) qa[(1 + v) * N + l] = ra3 * qa[(1 + v) * N + l] - fctr * umf[v];
-  double q1 = qa[l], q2 = qa[N + l], q3 = qa[2 * N + l], q4 = qa[3 * N + l];
-  const double q[5] = {q1, q2, q3, q4, rp * qa[4 * N + l] + ra2 * (ra0 * q1 + 0.5 * (q2 * q2 + q3 * q3 + q4 * q4) / q1)};
-  qa[4 * N + l] = q[4];
-  if (a.opt) put_primitives(b, c, ph, l, q);   // the next stage's primitives, formed in the update
+  const int l = indx3(b, ip * (b.L[d] - 1), j, k, d);
+  double q[5];
+  for (int v = 0; v < 5; v++) q[v] = b.qa[(size_t)v * N + l];
+  wall_state(a.coef[b.cs], phys(), b.nbc[d][ip], b.rpex[b.wall_off[d][ip] + jk], a.sc + b.cs * S_STRIDE + S_UMF1, q);
+  for (int v = 1; v < 5; v++) b.qa[(size_t)v * N + l] = q[v];
 }
 
 // ---- junction averaging, SingleTurbulence3D.f90:378-443 ----
