@@ -236,7 +236,8 @@ int32_t tp_sync(tp_context *ctx);
  * TP_OPT_CHUNKS = P (1 to 16) fixes the chunks per line of the
  *   chunked sweeps for every block and direction whose lines L allow chunks
  *   of ceil(L/P) <= 32 points; 0 (default) lets the library choose per block
- *   and direction.  The chunk count of a block depends only on its own line
+ *   and direction.  Lines of 513 to 1024 points are cut into chunks of at most
+ *   24 points whatever P is; longer ones run the sequential sweep.  The chunk count of a block depends only on its own line
  *   lengths (and on the autotuner's choice for its line-length class), so a
  *   case computes bit-identical results alone or batched with others when
  *   the chunk counts are fixed or left at their defaults.
@@ -258,12 +259,14 @@ int32_t tp_get_option(tp_context *ctx, int32_t option, int64_t *value);
  * count share a launch), five fields per launch as a time step runs them.
  * Overwrites the stage scratch (the flux and gradient work array), so call
  * it between steps.  chosen[d*2+kind] (kind 0 deriv, 1 filter) receives the
- * chunk count used for the most points (0: sequential kernel), us[d*2+kind]
+ * chunk count used for the most points (0: sequential kernel, or lines of
+ * more than 512 points), us[d*2+kind]
  * the time of the direction's launches; either may be NULL.  No counterpart
  * in the reference: it replaces the fixed 1-D loop structure of deriv/filte
  * with a measured launch shape. */
 int32_t tp_autotune(tp_context *ctx, int32_t reps, int32_t *chosen, double *us);
-/* chunks per line used for the most points, [d*2+kind] (0: sequential kernel) */
+/* chunks per line used for the most points, [d*2+kind] (0: sequential kernel,
+ * or lines of more than 512 points) */
 int32_t tp_col_config(tp_context *ctx, int32_t *chunks6);
 
 /* ---- turbulent inflow ----

@@ -291,27 +291,31 @@ void closure_rows(double fk, CaseCoef &c) {
 // l1 = -1, l2 = 0 and u1 = u2 = 0, u3 = -1: with a zero right-hand side such
 // a row only swaps the two carried values, exactly, so the sweeps run over
 // the whole capacity without selects (see fwd_sweep / bwd_sweep).
+// Long lines (lng, P up to COL_LONG_Q): 4 COL_LONG_Q doubles of either maps,
+// then per chunk runs of COL_LONG_C doubles l1, l2, u1, u2, u3, as the kernel's
+// LDS holds them.
 std::vector<double> col_tables(int L, int P, const double *l1, const double *l2, const double *u1,
-                               const double *u2, const double *u3) {
+                               const double *u2, const double *u3, bool lng = false) {
   const int Cl = (L + P - 1) / P, Pe = (L + Cl - 1) / Cl;
-  std::vector<double> T(128 + 192 * (size_t)Pe, 0.0);
+  const int S = lng ? COL_LONG_C : 32, M = lng ? 4 * COL_LONG_Q : 64, per = lng ? COL_LONG_F : 192;
+  std::vector<double> T(2 * M + (size_t)per * Pe, 0.0);
   auto L1 = [&](int i) { return i < 2 ? 0.0 : l1[i]; };
   auto L2 = [&](int i) { return i < 1 ? 0.0 : l2[i]; };
   auto U2 = [&](int i) { return i >= L - 1 ? 0.0 : u2[i]; };
   auto U3 = [&](int i) { return i >= L - 2 ? 0.0 : u3[i]; };
   for (int q = 0; q < Pe; q++) {
     const int s0 = q * Cl, e = std::min(L, s0 + Cl);
-    double *F = &T[128 + 192 * (size_t)q];
+    double *F = &T[2 * M + (size_t)per * q];
     for (int i = s0; i < e; i++) {
       const int k = i - s0;
-      F[k] = L1(i); F[32 + k] = L2(i);
-      F[64 + k] = u1[i]; F[96 + k] = U2(i);
-      F[128 + k] = U3(i);
+      F[k] = L1(i); F[S + k] = L2(i);
+      F[2 * S + k] = u1[i]; F[3 * S + k] = U2(i);
+      F[4 * S + k] = U3(i);
     }
-    for (int k = e - s0; k < 32; k++) {
-      F[k] = -1.0; F[32 + k] = 0.0;
-      F[64 + k] = 0.0; F[96 + k] = 0.0;
-      F[128 + k] = -1.0;
+    for (int k = e - s0; k < S; k++) {
+      F[k] = -1.0; F[S + k] = 0.0;
+      F[2 * S + k] = 0.0; F[3 * S + k] = 0.0;
+      F[4 * S + k] = -1.0;
     }
     for (int which = 0; which < 2; which++) {
       double ym2 = which == 0 ? 1 : 0, ym1 = which == 0 ? 0 : 1;
@@ -326,8 +330,8 @@ std::vector<double> col_tables(int L, int P, const double *l1, const double *l2,
         const double x = -U2(i) * xp1 - U3(i) * xp2;
         xp2 = xp1; xp1 = x;
       }
-      T[64 + 4 * q + which] = xp1;
-      T[64 + 4 * q + 2 + which] = xp2;
+      T[M + 4 * q + which] = xp1;
+      T[M + 4 * q + 2 + which] = xp2;
     }
   }
   return T;
@@ -352,13 +356,33 @@ size_t col_table_doubles(int L, int P) {
   return (128 + 192 * (size_t)Pe + 15) / 16 * 16;
 }
 
+// Waves of the line solves of a line longer than 16 chunks hold (512 points),
+// up to COL_LONG_MAX points; 0 for other lines.  They take COL_LONG_G chunks in
+// each wave, the fewest waves of full chunks (k_col).  701-point xi lines,
+// 1.3 M points, a launch of 4.5 fields on average: sequential 310 us, 16 waves
+// of 11-point chunks 79, 11 of 16 71, 8 of 22 71.  Up to 512 points one chunk a
+// wave is the better one: 241-point xi lines of 9 M points 201 us against 250,
+// 201-point eta lines of 20 M points 432 against 626, a 1 M-point case 1.60
+// ms a step against 1.76 (401-point xi lines 37 against 43).
+int long_waves(int L) {
+  if (L <= 512 || L > COL_LONG_MAX) return 0;
+  return (L + COL_LONG_G * COL_LONG_C - 1) / (COL_LONG_G * COL_LONG_C);
+}
+int long_chunk(int L) { return (L + COL_LONG_G * long_waves(L) - 1) / (COL_LONG_G * long_waves(L)); }
+size_t long_table_doubles(int L) {
+  const int Cl = long_chunk(L), Pe = (L + Cl - 1) / Cl;
+  return (8 * COL_LONG_Q + (size_t)COL_LONG_F * Pe + 15) / 16 * 16;
+}
+
 // doubles of all chunked-solver tables of a block with lines L[3]: every
 // chunk count its lines allow, both kinds
 size_t col_block_doubles(const int *L) {
   size_t n = 0;
-  for (int d = 0; d < 3; d++)
+  for (int d = 0; d < 3; d++) {
     for (int P : kColP)
       if (col_chunk(L[d], P)) n += 2 * col_table_doubles(L[d], P);
+    if (long_waves(L[d])) n += 2 * long_table_doubles(L[d]);
+  }
   return n;
 }
 
@@ -383,7 +407,7 @@ int col_default(int L, bool closure) {
   return 0;
 }
 
-// index of a chunk count in {0 (sequential), kColP...}: the line-length class
+// index of a chunk count in {0 (sequential or long lines), kColP...}: the line-length class
 // of blocks whose default is that count
 int col_class(int P) {
   for (int i = 0; i < kNColP; i++)
@@ -431,6 +455,7 @@ struct Mem {
 };
 
 // chunked-solver tables of one block: direction x kind x chunk-count index
+// (a long line's only table in the first place)
 using ColTab = std::array<const double *, 3 * 2 * kNColP>;
 
 struct HostCase {
@@ -467,7 +492,7 @@ struct DevList {
 // one launch of the line solves of a direction and kind: the blocks whose
 // lines use P chunks (P = 0: the sequential kernel) of capacity C points
 struct ColGroup {
-  int P = 0, C = 0;
+  int P = 0, C = 0, G = 1;
   bool closure = false;   // a block of the group has a closure face in this direction
   long long npts = 0;
   DevList work;
@@ -691,7 +716,7 @@ void run_line(tp_context *c, int kind, int d, int in_arr, int in_col, int out_ar
     a.work = g.work.d;
     a.direct = direct && g.closure ? 1 : 0;
     hipEvent_t e0 = t.start(i), e1 = t.stop(i, ng);
-    if (g.P) launch_col(d, kind, g.C, g.P, g.work.n, nf, c->stream, a, e0, e1);
+    if (g.P) launch_col(d, kind, g.C, g.P, g.G, g.work.n, nf, c->stream, a, e0, e1);
     else if (kind == 0) launch_deriv(d, g.work.n, nf, c->lds[d], c->stream, a, e0, e1);
     else launch_filter(d, g.work.n, nf, c->lds[d], c->stream, a, e0, e1);
     i++;
@@ -726,8 +751,9 @@ void choose_lines(tp_context *c) {
     const auto &src = c->bsrc[g];
     for (int d = 0; d < 3; d++)
       for (int kind = 0; kind < 2; kind++) {
-        const int P = block_chunks(c, (int)g, d, kind), ci = col_class(P) - 1;
-        c->blocks[g].colP[d][kind] = P;
+        const int P = block_chunks(c, (int)g, d, kind), W = long_waves(c->blocks[g].L[d]);
+        const int ci = W ? 0 : col_class(P) - 1;
+        c->blocks[g].colP[d][kind] = W ? W : P;
         c->blocks[g].col[d][kind] =
             ci < 0 ? nullptr : c->cases[src.first].coltab[src.second][(d * 2 + kind) * kNColP + ci];
       }
@@ -763,7 +789,8 @@ void merge_groups(std::vector<ColGroup> &groups, std::vector<std::vector<Work>> 
     again = false;
     for (size_t i = 0; i < groups.size() && !again; i++)
       for (size_t k = 0; k < groups.size() && !again; k++) {
-        if (i == k || !groups[i].P || !groups[k].P || waves(k, groups[k].P) > waves(i, groups[i].P)) continue;
+        if (i == k || !groups[i].P || !groups[k].P || groups[i].G != groups[k].G) continue;
+        if (waves(k, groups[k].P) > waves(i, groups[i].P)) continue;
         const int P = std::max(groups[i].P, groups[k].P);
         const bool both = waves(i, P) + waves(k, P) <= 8 * kSlots;
         const bool tail = groups[i].P == groups[k].P && groups[k].C <= groups[i].C && waves(k, P) <= kSlots;
@@ -784,24 +811,26 @@ int make_groups(tp_context *c, const std::vector<int> &gs, Mem &m, ListSet &L) {
       std::vector<std::vector<Work>> works;
       for (int g : gs) {
         const Block &b = c->blocks[g];
-        const int P = block_chunks(c, g, d, kind);
-        const int C = P ? col_capacity((b.L[d] + P - 1) / P) : 0;
+        const int W = long_waves(b.L[d]), G = W ? COL_LONG_G : 1;
+        const int P = W ? W : block_chunks(c, g, d, kind);
+        const int C = W ? COL_LONG_C : P ? col_capacity((b.L[d] + P - 1) / P) : 0;
         // a chunked launch reads the block's carry-map and factor table
         if (P && (!C || !b.col[d][kind]))
           return fail(TP_E_STATE, "block " + std::to_string(g) + " direction " + std::to_string(d + 1) +
                                       ": no chunked-solver table for " + std::to_string(P) + " chunks");
         size_t k = 0;
-        while (k < groups.size() && (groups[k].P != P || groups[k].C != C)) k++;
+        while (k < groups.size() && (groups[k].P != P || groups[k].C != C || groups[k].G != G)) k++;
         if (k == groups.size()) {
           groups.emplace_back();
           groups.back().P = P;
           groups.back().C = C;
+          groups.back().G = G;
           works.emplace_back();
         }
         for (int ip = 0; ip < 2; ip++)
           if (b.ndf[d][ip]) groups[k].closure = true;
         const int nlines = b.N / b.L[d];
-        const int step = P ? 64 : c->nlp[d] - 1;
+        const int step = P ? 64 / G : c->nlp[d] - 1;
         for (int q = 0; q < nlines; q += step) works[k].push_back({g, q, std::min(step, nlines - q), d});
         groups[k].npts += b.N;
       }
@@ -849,7 +878,7 @@ int make_groups(tp_context *c, const std::vector<int> &gs, Mem &m, ListSet &L) {
 // the chunk count that covers the most points (0: the sequential kernel)
 int top_chunks(const tp_context *c, int d, int kind) {
   long long n[17] = {0};
-  for (const Block &b : c->blocks) n[b.colP[d][kind]] += b.N;
+  for (const Block &b : c->blocks) n[long_waves(b.L[d]) ? 0 : b.colP[d][kind]] += b.N;
   return (int)(std::max_element(n, n + 17) - n);
 }
 
@@ -1382,6 +1411,14 @@ int build_case(HostCase &h) {
             T.resize(col_table_doubles(L, kColP[pi]), 0.0);
             all.insert(all.end(), T.begin(), T.end());
           }
+        }
+        for (int kind = 0; kind < 2 && long_waves(L); kind++) {
+          const std::vector<double> &lu = kind == 0 ? lud : luf;
+          std::vector<double> T = col_tables(L, COL_LONG_G * long_waves(L), &lu[0 * nl + o], &lu[1 * nl + o],
+                                             &lu[2 * nl + o], &lu[3 * nl + o], &lu[4 * nl + o], true);
+          slot.push_back({(d * 2 + kind) * kNColP, all.size()});
+          T.resize(long_table_doubles(L), 0.0);
+          all.insert(all.end(), T.begin(), T.end());
         }
       }
       double *dptr = nullptr;
@@ -2939,7 +2976,7 @@ int field_launch(FieldCall &f, char *ws, hipStream_t st) {
   a.m = 0; a.acc = 0; a.nlp = 65; a.copy_arr = -1;
   a.direct = f.periodic ? 1 : 0;   // periodic: closure sums from the other end of the same lines
   a.n45 = 0;
-  launch_col(f.d, 0, f.C, f.P, f.nwork, 1, st, a);
+  launch_col(f.d, 0, f.C, f.P, 1, f.nwork, 1, st, a);
   HIPCHK(hipGetLastError());
   return 0;
 }

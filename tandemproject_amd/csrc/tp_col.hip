@@ -191,12 +191,17 @@ __device__ inline double filter_bnd_row(const Block &b, const CaseCoef &c, int D
 
 
 constexpr int COL_TR = 65;   // row pitch (doubles) of the xi transpose buffer
+constexpr int COL_REACH = 160;  // points beyond which a carry has died out (long lines)
 constexpr int COL_DECAY = 48;  // points a carry travels sequentially before an amplifying closure
 
+// doubles of one chunk's factors in LDS: the table's own [6][32], or a long
+// line's five runs
+__host__ __device__ constexpr int col_fac(int G) { return G == 1 ? 192 : COL_LONG_F; }
+
 // dynamic LDS of a k_col launch, in doubles: carry pairs [2][P][64] (double2),
-// chunk factors [P][192], and for xi the transposes [P][8][COL_TR]
-__host__ __device__ constexpr int col_lds_doubles(int d, int P) {
-  return 2 * P * 64 * 2 + P * 192 + (d == 0 ? P * 8 * COL_TR : 0);
+// chunk factors, and for xi the transposes [P][8][COL_TR]
+__host__ __device__ constexpr int col_lds_doubles(int d, int P, int G) {
+  return 2 * P * 64 * 2 + P * G * col_fac(G) + (d == 0 ? P * 8 * COL_TR : 0);
 }
 
 // a zero the optimiser cannot see through: offsetting the factor pointer by
@@ -223,8 +228,9 @@ __device__ inline double lane_val(double v, int l) {
 }
 
 // Factors of the chunk's rows, copied to the wave's LDS slice:
-// F[k] = l1, F[32+k] = l2, F[64+k] = u1, F[96+k] = u2, F[128+k] = u3 of row
-// k.  Every lane reads the same address (an LDS broadcast).
+// F[k] = l1, F[S+k] = l2, F[2S+k] = u1, F[3S+k] = u2, F[4S+k] = u3 of row
+// k.  Every lane of the chunk reads the same address (an LDS broadcast).
+template <int S>
 struct ChunkLU {
   const double *F;
 };
@@ -235,14 +241,14 @@ struct ChunkLU {
 // carried pair exactly (y = 0 + ym2 - 0), so after them the pair is the one
 // of row n-1, swapped once more if their count is odd.  The opaque offset
 // keeps each sweep's factor loads inside the sweep.
-template <int C>
-__device__ inline void fwd_sweep(double (&r)[C], int n, const ChunkLU &f, double &ym2, double &ym1,
+template <int C, int S>
+__device__ inline void fwd_sweep(double (&r)[C], int n, const ChunkLU<S> &f, double &ym2, double &ym1,
                                  bool store) {
   const double *F = f.F + opaque_zero();
 #pragma unroll
   for (int k = 0; k < C; k++) {
     const double f1 = F[k];
-    const double f2 = F[32 + k];
+    const double f2 = F[S + k];
     const double y = r[k] - f1 * ym2 - f2 * ym1;
     if (store) r[k] = y;
     ym2 = ym1;
@@ -258,8 +264,8 @@ __device__ inline void fwd_sweep(double (&r)[C], int n, const ChunkLU &f, double
 // backward substitution from the carry (xp1, xp2) = (x[e+1], x[e+2]): the
 // padding rows k >= n come first, each swapping the pair (u1 = u2 = 0,
 // u3 = -1), so the carry enters them pre-swapped when their count is odd
-template <int C>
-__device__ inline void bwd_sweep(double (&r)[C], int n, const ChunkLU &f, double &xp1, double &xp2,
+template <int C, int S>
+__device__ inline void bwd_sweep(double (&r)[C], int n, const ChunkLU<S> &f, double &xp1, double &xp2,
                                  bool store) {
   const double *F = f.F + opaque_zero();
   if ((C - n) & 1) {
@@ -269,9 +275,9 @@ __device__ inline void bwd_sweep(double (&r)[C], int n, const ChunkLU &f, double
   }
 #pragma unroll
   for (int k = C - 1; k >= 0; k--) {
-    const double g1 = F[64 + k];
-    const double g2 = F[96 + k];
-    const double g3 = F[128 + k];
+    const double g1 = F[2 * S + k];
+    const double g2 = F[3 * S + k];
+    const double g3 = F[4 * S + k];
     const double x = g1 * r[k] - g2 * xp1 - g3 * xp2;
     if (store) r[k] = x;
     xp2 = xp1;
@@ -281,44 +287,73 @@ __device__ inline void bwd_sweep(double (&r)[C], int n, const ChunkLU &f, double
 
 // DIRECT: the launch forms the closure sums itself (a.direct) instead of
 // reading the exchange's recv slots
-template <int D, int KIND, int C, bool DIRECT>
+// G: chunks side by side in a wave.  1: the wave's 64 lanes are 64 lines.
+// COL_LONG_G, for lines longer than 16 waves of the largest chunks hold: 64 / G
+// lines in G lane groups, each group the next chunk of the same lines, so that
+// P waves hold G P chunks and the windows of a line still fit the registers.
+template <int D, int KIND, int C, bool DIRECT, int G>
 __global__ void __launch_bounds__(1024) k_col(LineArgs a) {
   extern __shared__ double lds[];
   const Work w = a.work[xcd_item(blockIdx.x, gridDim.x)];
   const Block &b = a.blocks[w.blk];
   const CaseCoef &c = a.coef[b.cs];
   const int L = b.L[D];
-  const int P = b.colP[D][KIND];                  // chunks of this block's lines
-  const int PL = blockDim.x >> 6;                 // waves of the launch, at least P
-  const int p = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  constexpr int NL = 64 / G, FS = G == 1 ? 32 : C, FC = col_fac(G);
+  const int P = G * b.colP[D][KIND];              // chunks of this block's lines
+  const int PL = blockDim.x >> 6;                 // waves of the launch, G of them hold at least P chunks
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
+  const int p = G == 1 ? wv : wv * G + lane / NL; // this lane's chunk
+  const int li = lane % NL;                       // and line
   const int Cl = (L + P - 1) / P;
   const int Pe = (L + Cl - 1) / Cl;               // chunks holding points
   const int s0 = p * Cl;
-  const int n = p < Pe ? min(Cl, L - s0) : 0;     // points of this wave's chunk
+  const int n = p < Pe ? min(Cl, L - s0) : 0;     // points of this lane's chunk
   const int nl = w.n;
-  const bool act = lane < nl;
+  const bool act = li < nl;
   const int stride = D == 0 ? 1 : D == 1 ? b.nx : b.nx * b.ny;
   int base, jk;
-  col_line<D>(b, w.a + (act ? lane : 0), base, jk);
+  col_line<D>(b, w.a + (act ? li : 0), base, jk);
   const int fi = blockIdx.y;   // field of a merged launch
   const double *src = field_ptr(b, a.in_arr, a.in_col + fi * a.in_step);
   double *dst = field_ptr(b, a.out_arr, a.out_col + fi * a.out_step);
   const double *rcv = b.recv[D] + (size_t)fi * 6 * b.F[D];
   const int mcap = a.m > 0 ? a.m + fi : 0;
-  double2 *pairA = reinterpret_cast<double2 *>(lds);      // [PL][64] carry-map inputs
-  double2 *pairB = pairA + PL * 64;                       // [PL][64] pairs handed along a chain
-  double *fl = reinterpret_cast<double *>(pairB + PL * 64) + p * 192;  // [PL][192] chunk factors
-  double *tr = reinterpret_cast<double *>(pairB + PL * 64) + PL * 192 + p * (8 * COL_TR);
+  double2 *pairA = reinterpret_cast<double2 *>(lds);      // [chunk][NL] carry-map inputs
+  double2 *pairB = pairA + PL * 64;                       // [chunk][NL] pairs handed along a chain
+  double *fw = reinterpret_cast<double *>(pairB + PL * 64) + wv * G * FC;   // the wave's chunk factors
+  double *tr = reinterpret_cast<double *>(pairB + PL * 64) + PL * G * FC + wv * (8 * COL_TR);
   const double *T = b.col[D][KIND];
-  const double mapf = T[lane], mapb = T[64 + lane];   // carry maps of all chunks
-  ChunkLU f;
-  {
-    const double *F = T + 128 + 192 * min(p, Pe - 1);
-    fl[lane] = F[lane]; fl[64 + lane] = F[64 + lane]; fl[128 + lane] = F[128 + lane];
-    f.F = fl;
-    wave_sync();   // the wave's own LDS writes precede its reads in issue order
+  // carry maps: of all chunks (G = 1), or of the window of chunks that this
+  // wave composes: a carry decays by 0.74 per point, so what comes from more
+  // than COL_REACH points away is below 1e-20 of it
+  const int reach = G == 1 ? 0 : (COL_REACH + Cl - 1) / Cl;
+  const int qf0 = G == 1 ? 0 : max(0, wv * G - reach), qb0 = G == 1 ? 0 : wv * G;
+  double mapf[G == 1 ? 1 : 2], mapb[G == 1 ? 1 : 2];
+  if (G == 1) {
+    mapf[0] = T[lane];
+    mapb[0] = T[64 + lane];
+  } else {
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+      mapf[G == 1 ? 0 : h] = T[4 * qf0 + 64 * h + lane];
+      mapb[G == 1 ? 0 : h] = T[4 * COL_LONG_Q + 4 * qb0 + 64 * h + lane];
+    }
   }
+  ChunkLU<FS> f;
+  if (G == 1) {
+    const double *F = T + 128 + 192 * min(p, Pe - 1);
+    fw[lane] = F[lane]; fw[64 + lane] = F[64 + lane]; fw[128 + lane] = F[128 + lane];
+    f.F = fw;
+  } else {
+    // the tables' chunks are laid out as the LDS holds them
+    for (int g = 0; g < G; g++) {
+      const double *F = T + 8 * COL_LONG_Q + (size_t)FC * min(wv * G + g, Pe - 1);
+      for (int k = lane; k < 5 * C; k += 64) fw[g * FC + k] = F[k];
+    }
+    f.F = fw + (lane / NL) * FC;
+  }
+  wave_sync();   // the wave's own LDS writes precede its reads in issue order
 
   // Chains at one-sided closures.  End: the last Rhi chunks take their
   // forward carry from the chunk before them, one after the other.  Start:
@@ -367,7 +402,7 @@ __global__ void __launch_bounds__(1024) k_col(LineArgs a) {
   // ---- window rows s0-3 .. s0+n+2, clamped to the line; the rows of the
   // capacity padding past them are not read (zero) ----
   double v[C + 6];
-  const int nw = n + 6;   // window rows in use
+  const int nw = (D == 0 && G > 1 ? Cl : n) + 6;   // window rows in use
   if (D == 0) {
     // all global loads of the window first (8 lines x 8 consecutive points per
     // instruction), then the transposes through LDS piece by piece
@@ -375,10 +410,13 @@ __global__ void __launch_bounds__(1024) k_col(LineArgs a) {
     double tmp[NPC][8];
 #pragma unroll
     for (int t = 0; t < NPC; t++) {
-      const int row = min(max(s0 - 3 + 8 * t + (lane & 7), 0), L - 1);
 #pragma unroll
       for (int j = 0; j < 8; j++) {
-        const int rl = min((lane >> 3) + 8 * j, nl - 1);
+        // the (chunk, line) of lane 8j + lane / 8
+        const int q = (lane >> 3) + 8 * j;
+        const int sq = G == 1 ? s0 : (wv * G + q / NL) * Cl;
+        const int row = min(max(sq - 3 + 8 * t + (lane & 7), 0), L - 1);
+        const int rl = min(q % NL, nl - 1);
         tmp[t][j] = 8 * t < nw ? at(src, 8u * (unsigned)((w.a + rl) * b.nx + row)) : 0.0;
       }
     }
@@ -521,27 +559,30 @@ __global__ void __launch_bounds__(1024) k_col(LineArgs a) {
   // ---- forward substitution ----
   double ym2 = 0.0, ym1 = 0.0;
   fwd_sweep<C>(r, n, f, ym2, ym1, false);
-  pairA[p * 64 + lane] = make_double2(ym2, ym1);
+  pairA[p * NL + li] = make_double2(ym2, ym1);
   __syncthreads();
   double c0 = 0.0, c1 = 0.0;
-  for (int q = 0; q < min(p, Pe); q++) {
-    const double m0 = lane_val(mapf, 4 * q), m1 = lane_val(mapf, 4 * q + 1);
-    const double m2 = lane_val(mapf, 4 * q + 2), m3 = lane_val(mapf, 4 * q + 3);
-    const double2 e = pairA[q * 64 + lane];
+  const int qfe = min(G == 1 ? p : wv * G + G - 1, Pe);
+  for (int q = qf0; q < qfe; q++) {
+    const double mq = G == 1 || q - qf0 < 16 ? mapf[0] : mapf[G == 1 ? 0 : 1];
+    const int at = 4 * (G == 1 ? q : (q - qf0) & 15);
+    const double m0 = lane_val(mq, at), m1 = lane_val(mq, at + 1);
+    const double m2 = lane_val(mq, at + 2), m3 = lane_val(mq, at + 3);
+    const double2 e = pairA[q * NL + li];
     const double t0 = m0 * c0 + m1 * c1 + e.x;
     const double t1 = m2 * c0 + m3 * c1 + e.y;
-    c0 = t0; c1 = t1;
+    if (G == 1 || q < p) { c0 = t0; c1 = t1; }
   }
   for (int t = 0; t <= Tf; t++) {
     if (t > 0) __syncthreads();
     if (tf == t) {
       if (t > 0) {
-        const double2 e = pairB[(p - 1) * 64 + lane];
+        const double2 e = pairB[(p - 1) * NL + li];
         c0 = e.x; c1 = e.y;
       }
       ym2 = c0; ym1 = c1;
       fwd_sweep<C>(r, n, f, ym2, ym1, true);
-      pairB[p * 64 + lane] = make_double2(ym2, ym1);
+      pairB[p * NL + li] = make_double2(ym2, ym1);
     }
   }
   __syncthreads();   // every wave has read pairA and pairB before they are reused
@@ -549,27 +590,30 @@ __global__ void __launch_bounds__(1024) k_col(LineArgs a) {
   // ---- backward substitution ----
   double xp1 = 0.0, xp2 = 0.0;
   bwd_sweep<C>(r, n, f, xp1, xp2, false);
-  pairA[p * 64 + lane] = make_double2(xp1, xp2);
+  pairA[p * NL + li] = make_double2(xp1, xp2);
   __syncthreads();
   double d0 = 0.0, d1 = 0.0;
-  for (int q = Pe - 1; q > p; q--) {
-    const double m0 = lane_val(mapb, 4 * q), m1 = lane_val(mapb, 4 * q + 1);
-    const double m2 = lane_val(mapb, 4 * q + 2), m3 = lane_val(mapb, 4 * q + 3);
-    const double2 e = pairA[q * 64 + lane];
+  const int qbe = G == 1 ? p : qb0;
+  for (int q = G == 1 ? Pe - 1 : min(Pe - 1, qb0 + G - 1 + reach); q > qbe; q--) {
+    const double mq = G == 1 || q - qb0 < 16 ? mapb[0] : mapb[G == 1 ? 0 : 1];
+    const int at = 4 * (G == 1 ? q : (q - qb0) & 15);
+    const double m0 = lane_val(mq, at), m1 = lane_val(mq, at + 1);
+    const double m2 = lane_val(mq, at + 2), m3 = lane_val(mq, at + 3);
+    const double2 e = pairA[q * NL + li];
     const double t0 = m0 * d0 + m1 * d1 + e.x;
     const double t1 = m2 * d0 + m3 * d1 + e.y;
-    d0 = t0; d1 = t1;
+    if (G == 1 || q > p) { d0 = t0; d1 = t1; }
   }
   for (int t = 0; t <= Tb; t++) {
     if (t > 0) __syncthreads();
     if (tb == t) {
       if (t > 0) {
-        const double2 e = pairB[(p + 1) * 64 + lane];
+        const double2 e = pairB[(p + 1) * NL + li];
         d0 = e.x; d1 = e.y;
       }
       xp1 = d0; xp2 = d1;
       bwd_sweep<C>(r, n, f, xp1, xp2, true);
-      pairB[p * 64 + lane] = make_double2(xp1, xp2);
+      pairB[p * NL + li] = make_double2(xp1, xp2);
     }
   }
 
@@ -596,14 +640,14 @@ __global__ void __launch_bounds__(1024) k_col(LineArgs a) {
   // workgroup stores them as one run of whole cache lines: a wave's own
   // pieces (8 rows x 8 points) would straddle 64-byte write granules.
   const int pitch = L + 1;
-  int R = 64;
-  while (R >= 8 && R * pitch > col_lds_doubles(0, PL)) R >>= 1;
-  if (D == 0 && R >= 8) {
+  int R = NL;
+  while (R >= (G == 1 ? 8 : 2) && R * pitch > col_lds_doubles(0, PL, G)) R >>= 1;
+  if (D == 0 && (G > 1 || R >= 8)) {
     double *tile = lds;
     __syncthreads();
     for (int h = 0; h * R < nl; h++) {
-      if (act && lane >= h * R && lane < (h + 1) * R) {
-        double *trow = tile + (lane - h * R) * pitch + s0;
+      if (act && li >= h * R && li < (h + 1) * R) {
+        double *trow = tile + (li - h * R) * pitch + s0;
 #pragma unroll
         for (int k = 0; k < C; k++)
           if (k < n) trow[k] = r[k];
@@ -696,19 +740,28 @@ __global__ void __launch_bounds__(1024) k_col(LineArgs a) {
   }
 }
 
-size_t col_lds_bytes(int d, int P) { return (size_t)col_lds_doubles(d, P) * sizeof(double); }
+size_t col_lds_bytes(int d, int P, int G) { return (size_t)col_lds_doubles(d, P, G) * sizeof(double); }
+
+template <int D, int KIND>
+static void launch_long(int P, int nwg, int nf, hipStream_t st, const LineArgs &a, hipEvent_t e0, hipEvent_t e1) {
+  const size_t lds = col_lds_bytes(D, P, COL_LONG_G);
+  if (KIND == 0 && a.direct)
+    TP_LAUNCH_EV((k_col<D, KIND, COL_LONG_C, KIND == 0, COL_LONG_G>), dim3(nwg, nf), dim3(64 * P), lds, st, e0, e1, a);
+  else
+    TP_LAUNCH_EV((k_col<D, KIND, COL_LONG_C, false, COL_LONG_G>), dim3(nwg, nf), dim3(64 * P), lds, st, e0, e1, a);
+}
 
 template <int D, int KIND>
 static void launch_col_c(int C, int P, int nwg, int nf, hipStream_t st, const LineArgs &a, hipEvent_t e0,
                          hipEvent_t e1) {
-  const size_t lds = col_lds_bytes(D, P);
+  const size_t lds = col_lds_bytes(D, P, 1);
   switch (C) {
 #define CASE_C(CV)                                                                                     \
   case CV:                                                                                           \
     if (KIND == 0 && a.direct)                                                                       \
-      TP_LAUNCH_EV((k_col<D, KIND, CV, KIND == 0>), dim3(nwg, nf), dim3(64 * P), lds, st, e0, e1, a); \
+      TP_LAUNCH_EV((k_col<D, KIND, CV, KIND == 0, 1>), dim3(nwg, nf), dim3(64 * P), lds, st, e0, e1, a); \
     else                                                                                             \
-      TP_LAUNCH_EV((k_col<D, KIND, CV, false>), dim3(nwg, nf), dim3(64 * P), lds, st, e0, e1, a);    \
+      TP_LAUNCH_EV((k_col<D, KIND, CV, false, 1>), dim3(nwg, nf), dim3(64 * P), lds, st, e0, e1, a);    \
     break;
     CASE_C(8) CASE_C(12) CASE_C(16) CASE_C(20) CASE_C(24) CASE_C(28) CASE_C(32)
 #undef CASE_C
@@ -722,17 +775,20 @@ int col_capacity(int chunk) {
   return chunk <= 8 ? 8 : (chunk + 3) / 4 * 4;
 }
 
-void launch_col(int d, int kind, int C, int P, int nwg, int nf, hipStream_t st, const LineArgs &a, hipEvent_t e0,
-                hipEvent_t e1) {
-  if (kind == 0) {
-    if (d == 0) launch_col_c<0, 0>(C, P, nwg, nf, st, a, e0, e1);
-    else if (d == 1) launch_col_c<1, 0>(C, P, nwg, nf, st, a, e0, e1);
-    else launch_col_c<2, 0>(C, P, nwg, nf, st, a, e0, e1);
-  } else {
-    if (d == 0) launch_col_c<0, 1>(C, P, nwg, nf, st, a, e0, e1);
-    else if (d == 1) launch_col_c<1, 1>(C, P, nwg, nf, st, a, e0, e1);
-    else launch_col_c<2, 1>(C, P, nwg, nf, st, a, e0, e1);
+void launch_col(int d, int kind, int C, int P, int G, int nwg, int nf, hipStream_t st, const LineArgs &a,
+                hipEvent_t e0, hipEvent_t e1) {
+#define BY_KIND(D)                                                       \
+  if (G == 1) {                                                          \
+    if (kind == 0) launch_col_c<D, 0>(C, P, nwg, nf, st, a, e0, e1);     \
+    else launch_col_c<D, 1>(C, P, nwg, nf, st, a, e0, e1);               \
+  } else {                                                               \
+    if (kind == 0) launch_long<D, 0>(P, nwg, nf, st, a, e0, e1);    \
+    else launch_long<D, 1>(P, nwg, nf, st, a, e0, e1);              \
   }
+  if (d == 0) { BY_KIND(0) }
+  else if (d == 1) { BY_KIND(1) }
+  else { BY_KIND(2) }
+#undef BY_KIND
 }
 
 }  // namespace tp

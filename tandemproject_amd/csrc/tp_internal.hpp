@@ -21,6 +21,11 @@ constexpr int LMF = 8;    // filter closure length - 1
 constexpr int LMP = 11;
 constexpr int MBCI = 3;   // GCBC spreading depth
 constexpr int MAX_CASE = 4096;
+// chunked line solves of long lines: chunks side by side in a wave, their
+// capacity, the most chunks of a line and the longest such line; doubles of a
+// chunk's factors, padded so that the lane groups' reads of one row fall into
+// different LDS banks (2 x 120 = 48 modulo the 64 banks)
+constexpr int COL_LONG_G = 4, COL_LONG_C = 24, COL_LONG_Q = 44, COL_LONG_MAX = 1024, COL_LONG_F = 120;
 constexpr int RCV_SLOTS = 5;  // fields whose closure sums one exchange launch can hold
 
 // ---- per-case scalars on the device (src/MainVar3D.f90:139-142) ----
@@ -99,7 +104,8 @@ struct Block {
   double *snor;               // [3][nsurf] unit normals into the fluid (walldir)
   double *sst;                // [3][nsurf] previous sampled p, trapezoid integrals of p and p^2
   const double *col[3][2];    // chunked-solver carry maps per direction, kind (deriv, filter)
-  int colP[3][2];             // chunks per line they are for (0: the sequential kernel)
+  int colP[3][2];             // chunks per line they are for (0: the sequential kernel); in the
+                              // long-line layout waves, COL_LONG_G chunks each
 };
 
 // array ids exposed through the C ABI (order shared with include/tandem_hip.h)
@@ -277,13 +283,14 @@ void launch_inflow_table(const double *modes, const double *rot, int nmodes, con
                          double fctr, const double *uoo, double *vito, hipStream_t st);
 void launch_eddy_table(const double *eddies, int nits, const double *pos, int ng, int ntz, double fctr,
                        const double *uoo, double slit, double span, double cfit, double *vito, hipStream_t st);
-// chunked line solves: P waves per 64 lines, chunk capacity C points per lane
+// chunked line solves: P waves per 64 / G lines, G chunks per wave (1 or
+// COL_LONG_G), chunk capacity C points per lane
 int col_capacity(int chunk);
-size_t col_lds_bytes(int d, int P);
+size_t col_lds_bytes(int d, int P, int G);
 // e0, e1 (optional): timing events carried in the launch's own dispatch
 // (hipExtLaunchKernel), recorded as the kernel starts and ends, instead of
 // event packets of their own between the launches
-void launch_col(int d, int kind, int C, int P, int nwg, int nf, hipStream_t st, const LineArgs &a,
+void launch_col(int d, int kind, int C, int P, int G, int nwg, int nf, hipStream_t st, const LineArgs &a,
                 hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
 void launch_deriv(int d, int nwg, int nf, size_t lds, hipStream_t st, const LineArgs &a,
                   hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
