@@ -360,7 +360,7 @@ size_t col_table_doubles(int L, int P) {
 // up to COL_LONG_MAX points; 0 for other lines.  They take COL_LONG_G chunks in
 // each wave, the fewest waves of full chunks (k_col).  701-point xi lines,
 // 1.3 M points, a launch of 4.5 fields on average: sequential 310 us, 16 waves
-// of 11-point chunks 79, 11 of 16 71, 8 of 22 71.  Up to 512 points one chunk a
+// of 11-point chunks 79, 11 of 16 71, 8 of 22 54.  Up to 512 points one chunk a
 // wave is the better one: 241-point xi lines of 9 M points 201 us against 250,
 // 201-point eta lines of 20 M points 432 against 626, a 1 M-point case 1.60
 // ms a step against 1.76 (401-point xi lines 37 against 43).
@@ -502,6 +502,7 @@ struct ListSet {
   DevList points, sponge, force, lines[3], exch, gprep, gapply[3], wall, acap, normals;
   DevList surf;                     // wall-surface points, 256 per item
   std::vector<ColGroup> cg[3][2];   // line-solve launches per direction and kind
+  ColGroup dirs;                    // the derivatives' launches of all directions as one (P = 0: apart)
   std::vector<int> wr;   // first point-work item of each linked case, then the end
   std::vector<int> wwr;  // first wall-surface item of each linked case, then the end
 };
@@ -684,6 +685,18 @@ void run_exchange(tp_context *c, int nt, int nrt, int n45, int arr, int col0, in
   launch_exchange(L.n, nf, c->stream, a);
 }
 
+LineArgs line_args(tp_context *c, int in_arr, int in_col, int out_arr, int out_col, int m, int acc, int in_step,
+                   int out_step) {
+  LineArgs a;
+  std::memset(&a, 0, sizeof(a));
+  a.blocks = c->d_blocks; a.coef = c->d_coef;
+  a.in_arr = in_arr; a.in_col = in_col; a.out_arr = out_arr; a.out_col = out_col;
+  a.m = m; a.acc = acc;
+  a.in_step = in_step; a.out_step = out_step;
+  a.copy_arr = -1;
+  return a;
+}
+
 // line solves of direction d over nf fields in one launch: field f reads
 // column in_col + f in_step, writes out_col + f out_step, uses recv slot f
 // (filled by an exchange over the same fields) and captures drva column m + f
@@ -695,14 +708,10 @@ void run_line(tp_context *c, int kind, int d, int in_arr, int in_col, int out_ar
   // read, a copy of the output (the last filter's qo) also written
   Timed t(c, kind == 0 ? K_DERIV : K_FILTER, ((acc ? 24.0 : 16.0) + (copy_arr >= 0 ? 8.0 : 0.0)) * (double)c->npts * nf,
           true);
-  LineArgs a;
-  a.blocks = c->d_blocks; a.work = c->L.lines[d].d; a.coef = c->d_coef;
-  a.in_arr = in_arr; a.in_col = in_col; a.out_arr = out_arr; a.out_col = out_col;
-  a.m = m; a.acc = acc; a.nlp = c->nlp[d];
-  a.in_step = in_step; a.out_step = out_step;
+  LineArgs a = line_args(c, in_arr, in_col, out_arr, out_col, m, acc, in_step, out_step);
+  a.work = c->L.lines[d].d; a.nlp = c->nlp[d];
   a.copy_arr = copy_arr; a.copy_col = copy_col;
   a.direct = direct ? 1 : 0;
-  a.n45 = 0;
   if (c->exact_lines) {
     hipEvent_t e0 = t.start(0), e1 = t.stop(0, 1);
     if (kind == 0) launch_deriv(d, c->L.lines[d].n, nf, c->lds[d], c->stream, a, e0, e1);
@@ -805,6 +814,9 @@ void merge_groups(std::vector<ColGroup> &groups, std::vector<std::vector<Work>> 
 // line-solve launches over the global blocks gs: one per distinct chunk
 // count and chunk capacity of each direction and kind, small ones merged
 int make_groups(tp_context *c, const std::vector<int> &gs, Mem &m, ListSet &L) {
+  ColGroup dirs;
+  std::vector<Work> all;
+  bool one_each = true;
   for (int d = 0; d < 3; d++)
     for (int kind = 0; kind < 2; kind++) {
       std::vector<ColGroup> groups;
@@ -870,8 +882,29 @@ int make_groups(tp_context *c, const std::vector<int> &gs, Mem &m, ListSet &L) {
       }
       for (size_t k = 0; k < groups.size(); k++)
         if (int rc = upload_list(m, groups[k].work, works[k])) return rc;
+      if (kind == 0) {
+        one_each = one_each && groups.size() == 1 && groups[0].P && groups[0].P <= 8 && groups[0].G == 1 &&
+                   (d == 2 || !groups[0].closure);
+        if (one_each) {
+          dirs.P = std::max(dirs.P, groups[0].P);
+          dirs.C = std::max(dirs.C, groups[0].C);
+          dirs.npts += groups[0].npts;
+          all.insert(all.end(), works[0].begin(), works[0].end());
+        }
+      }
       L.cg[d][kind] = std::move(groups);
     }
+  // one launch for the gradients of all three directions while its waves (at the
+  // largest chunk count of the three) are at most half the GPU's slots: 28 k
+  // points 25 us as three launches, 13.7 as one; 49 k 31 and 16.6, 87 k (1.5 k
+  // waves) 33 and 22; beyond, idle waves and padding cost more than the
+  // launches: 129 k points (3.5 k waves) 36 and 39, 208 k 44 and 50
+  L.dirs = ColGroup();
+  if (one_each && !all.empty() && 4LL * dirs.P * (long long)all.size() <= kSlots / 2) {
+    dirs.C = dirs_capacity(dirs.C);
+    if (int rc = upload_list(m, dirs.work, all)) return rc;
+    L.dirs = dirs;
+  }
   return 0;
 }
 
@@ -960,6 +993,15 @@ void enqueue_begin(tp_context *c, int nk, bool prim_ready = false, bool lean = f
 void enqueue_gradients(tp_context *c) {
   if (!c->any_visc) return;
   const bool dir = direct_ok(c, 0);
+  if (dir && c->L.dirs.P) {
+    const ColGroup &g = c->L.dirs;
+    Timed t(c, K_DERIV, 16.0 * (double)c->npts * 12, true);
+    LineArgs a = line_args(c, F_DE, 1, F_FX, 0, 0, 0, 1, 3);
+    a.work = g.work.d;
+    hipEvent_t e0 = t.start(0), e1 = t.stop(0, 1);
+    launch_col_dirs(g.C, g.P, g.work.n, 4, c->stream, a, e0, e1);
+    return;
+  }
   if (!dir) run_exchange(c, 0, 1, 0, F_DE, 1, 4, 1);
   run_line(c, 0, 2, F_DE, 1, F_FX, 2, 0, 0, 4, 1, 3, -1, 0, dir);
   run_line(c, 0, 1, F_DE, 1, F_FX, 1, 0, 0, 4, 1, 3, -1, 0, dir);
