@@ -1075,15 +1075,17 @@ void enqueue_rk(tp_context *c, int nk, bool wall, bool prim = false, bool lean =
 void enqueue_wall(tp_context *c) { run_faces(c, c->L.wall, FK_WALL, base_args(c), K_GCBC); }
 
 // corner junctions, src/SingleTurbulence3D.f90:378-443
-void enqueue_junction(tp_context *c, bool prim = false) {
+void enqueue_junction(tp_context *c, bool prim = false, bool captured = false) {
   if (c->njct)
-    launch_junction(c->d_blocks, c->d_coef, c->d_jct, c->d_jvel, c->njct, c->maxk, prim ? 1 : 0, c->stream);
+    launch_junction(c->d_blocks, c->d_coef, c->d_jct, c->d_jvel, c->njct, c->maxk, prim ? 1 : 0,
+                    captured ? 1 : 0, c->stream);
 }
 
 // interface averaging, src/Main3D.f90:897-952
-void enqueue_avg(tp_context *c, bool prim = false) {
+// captured: the update and the junctions left the faces' states in drva
+void enqueue_avg(tp_context *c, bool prim = false, bool captured = false) {
   StageArgs a = base_args(c);
-  run_faces(c, c->L.acap, FK_AVG_CAP, a, K_GCBC);
+  if (!captured) run_faces(c, c->L.acap, FK_AVG_CAP, a, K_GCBC);
   a.opt = prim ? 1 : 0;
   run_faces(c, c->L.acap, FK_AVG_APPLY, a, K_GCBC);
 }
@@ -1109,8 +1111,8 @@ void enqueue_stage(tp_context *c, int nk, bool prim_ready = false, bool prim_nex
   enqueue_gcbc(c);
   c->qin = false;   // the update reads qo and writes qa in any case
   enqueue_rk(c, nk, true, prim_next, lean);
-  enqueue_junction(c, prim_next);
-  enqueue_avg(c, prim_next);
+  enqueue_junction(c, prim_next, true);
+  enqueue_avg(c, prim_next, true);
 }
 
 // a time step: the filter step, then the stages, each but the last leaving

@@ -268,7 +268,7 @@ struct StageArgs {
   double *part;      // reduction partials [nwork][2]
   double *wpart;     // wall-force partials [nwallwork][4]
   int nk, m, d, opt; // stage number, field, direction, option (k_flux_all: write tv everywhere;
-                     // k_rk: apply the wall conditions too; k_avg_apply: form the primitives
+                     // k_rk: the wall conditions and the averaging's captures too; k_avg_apply: form the primitives
                      // of the points it changes)
   int arr, col;      // generic field selector
   int o0, o1, o2;    // tv slots for gradient combination (-1..-3 = ss columns)
@@ -317,7 +317,7 @@ void launch_sc_dt(const CaseCoef *coef, double *sc, const double *part, const in
 void launch_sc_rk(const CaseCoef *coef, double *sc, int ncase, int nk, hipStream_t st);
 void launch_sc_end(const CaseCoef *coef, double *sc, int ncase, hipStream_t st);
 void launch_junction(const Block *blocks, const CaseCoef *coef, const int *jct, const int *jvel, int njct, int maxk,
-                     int prim, hipStream_t st);
+                     int prim, int cap, hipStream_t st);
 void launch_surf_reduce(const CaseCoef *coef, double *sc, const double *wpart, const int *wwr, int ncase,
                         hipStream_t st);
 

@@ -1058,12 +1058,29 @@ __device__ inline void wall_state(const CaseCoef &c, const Phys &ph, int np, dou
 
 __device__ inline bool wall_code(int np) { return np == 20 || np == 25; }
 
+// faces that the interface averaging works on (Main3D.f90:901-952)
+__device__ inline bool avg_code(int np) { return np == 30 || np == 35 || np == 45; }
+__device__ inline bool avg_face(const Block &b, const CaseCoef &c, int d, int ip) {
+  const int np = b.nbc[d][ip];
+  return avg_code(np) || (c.nextgcic == 1 && (np == 20 || np == 25));
+}
+
+// the state of a point on face (d, s), kept for the interface averaging
+__device__ inline void capture_face(const Block &b, int d, int s, int x, int y, int z, const double q[5]) {
+  const int F = b.F[d], jk = d == 0 ? z * b.ny + y : d == 1 ? x * b.nz + z : y * b.nx + x;
+#pragma unroll
+  for (int v = 0; v < 5; v++) b.drva[d][(s * 5 + v) * F + jk] = q[v];
+}
+
 // ---- RK update, Main3D.f90:876-881 ----
 // PRIM: also the next stage's primitives of the updated state (k_primitives'
 // arithmetic on the same values) that the stage reads, u, v, w, T into
 // de(:,2:5) and p, once the residual is read; the junction and averaging
 // passes that follow form them again at the points they change
-// opt: also the wall conditions at the points of wall faces, which need
+// opt: also each averaged face's state into drva, which a launch of its own
+// (k_avg_capture, still the averaging drop-in's) did after the junctions (5.2 us a
+// stage at 28 k points, 5.8 at 208 k, 7.1 at 1 M, 30 at 20 M; here 1, 1, 3 and 12;
+// the junctions rewrite theirs); and the wall conditions at the points of wall faces, which need
 // nothing but the point's own state (a launch of their own took 4.4 us a stage at 28 k
 // points and 6.0 at 20 M; the steps are 2.6 % shorter at 28 k and 1.2 % at 1 M
 // points, the same within 0.2 % at 20 M)
@@ -1074,18 +1091,22 @@ __global__ void __launch_bounds__(256) k_rk(StageArgs a) {
   const double dtk = sc[S_DTK];
   const CaseCoef &c = a.coef[b.cs];
   const Phys ph = phys();
-  bool walls = false;
+  bool walls = false, avgs = false;
   if (a.opt)
-    for (int d = 0; d < 3; d++) walls = walls || wall_code(b.nbc[d][0]) || wall_code(b.nbc[d][1]);
+    for (int d = 0; d < 3; d++)
+      for (int s = 0; s < 2; s++) {
+        walls = walls || wall_code(b.nbc[d][s]);
+        avgs = avgs || avg_face(b, c, d, s);
+      }
   for (int l = w.a + threadIdx.x; l < w.a + w.n; l += blockDim.x) {
     double r1 = dtk * ld_stream(&b.yaco[l]);
     double q[5];
     for (int v = 0; v < 5; v++)
       q[v] = ld_stream(&b.qo[(size_t)v * N + l]) - r1 * ld_stream(&b.de[(size_t)v * N + l]);
+    int x = 0, y = 0, z = 0;
+    if (walls || avgs) point_ijk(b, l, x, y, z);
+    const int idx[3] = {x, y, z};
     if (walls) {
-      int x, y, z;
-      point_ijk(b, l, x, y, z);
-      const int idx[3] = {x, y, z};
       for (int d = 0; d < 3; d++) {
         const int s = idx[d] == 0 ? 0 : 1;
         if ((idx[d] != 0 && idx[d] != b.L[d] - 1) || !wall_code(b.nbc[d][s])) continue;
@@ -1094,6 +1115,12 @@ __global__ void __launch_bounds__(256) k_rk(StageArgs a) {
       }
     }
     for (int v = 0; v < 5; v++) st_stream(&b.qa[(size_t)v * N + l], q[v]);
+    if (avgs) {
+      for (int d = 0; d < 3; d++) {
+        if (idx[d] == 0 && avg_face(b, c, d, 0)) capture_face(b, d, 0, x, y, z, q);
+        if (idx[d] == b.L[d] - 1 && avg_face(b, c, d, 1)) capture_face(b, d, 1, x, y, z, q);
+      }
+    }
     if (PRIM) {
       const Prim r = primitives(c, ph, q[0], q[1], q[2], q[3], q[4]);
       st_stream(&b.de[N + l], r.d2);
@@ -1122,39 +1149,53 @@ __global__ void __launch_bounds__(256) k_wall(StageArgs a) {
 }
 
 // ---- junction averaging, SingleTurbulence3D.f90:378-443 ----
-// jct[j*12 + mbr*3 + {block, ip, jp}], jvel[j*2 + {0,1}]; one thread per (junction, k)
+// jct[j*12 + mbr*3 + {block, ip, jp}], jvel[j*2 + {0,1}]; four threads per
+// (junction, k), one for each member: all read the four states, then each
+// writes its own corner (one thread for all four, a chain of their loads and
+// stores, took 6.3 us a launch at 28 k points and, with cap, 12.8; now 6.5)
 // prim: also the primitives of the new corner states (the next stage's,
-// formed in the update)
-__global__ void k_junction(const Block *blocks, const CaseCoef *coef, const int *jct, const int *jvel, int njct,
-                           int maxk, int prim) {
-  int t = blockIdx.x * blockDim.x + threadIdx.x;
-  int jn = t / maxk, k = t % maxk;
-  if (jn >= njct) return;
-  const int *J = jct + jn * 12;
-  if (k > blocks[J[0]].nz - 1) return;
-  double v[4][5];
-  int lq[4];
-  for (int q = 0; q < 4; q++) {
-    const Block &b = blocks[J[q * 3]];
-    int i = J[q * 3 + 1] * (b.nx - 1), j = J[q * 3 + 2] * (b.ny - 1);
-    lq[q] = indx3(b, i, j, k, 0);
-    for (int m = 0; m < 5; m++) v[q][m] = b.qa[(size_t)m * b.N + lq[q]];
+// formed in the update); cap: also the corners' states kept for the averaging
+__global__ void __launch_bounds__(64) k_junction(const Block *blocks, const CaseCoef *coef, const int *jct,
+                                                 const int *jvel, int njct, int maxk, int prim, int cap) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  const int q = t & 3, jn = (t >> 2) / maxk, k = (t >> 2) % maxk;
+  const int *J = jct + min(jn, njct - 1) * 12;
+  const bool on = jn < njct && k <= blocks[J[0]].nz - 1;
+  const int va = jvel[min(jn, njct - 1) * 2], vb = jvel[min(jn, njct - 1) * 2 + 1];
+  double v[4][5], r[5];
+  if (on) {
+#pragma unroll
+    for (int w = 0; w < 4; w++) {
+      const Block &b = blocks[J[w * 3]];
+      const int l = indx3(b, J[w * 3 + 1] * (b.nx - 1), J[w * 3 + 2] * (b.ny - 1), k, 0);
+#pragma unroll
+      for (int m = 0; m < 5; m++) v[w][m] = b.qa[(size_t)m * b.N + l];
+    }
+    // selects: an index known only at run time would send v to scratch memory
+    auto pick = [&](int w, int m) { return w == 0 ? v[0][m] : w == 1 ? v[1][m] : w == 2 ? v[2][m] : v[3][m]; };
+    r[0] = 0.25 * (v[0][0] + v[1][0] + v[2][0] + v[3][0]);
+#pragma unroll
+    for (int m = 1; m <= 3; m++) r[m] = 0.5 * (pick(va, m) + pick(vb, m));
+    r[4] = 0.25 * (v[0][4] + v[1][4] + v[2][4] + v[3][4]);
   }
-  int va = jvel[jn * 2], vb = jvel[jn * 2 + 1];
-  double r[5];
-  r[0] = 0.25 * (v[0][0] + v[1][0] + v[2][0] + v[3][0]);
-  for (int m = 1; m <= 3; m++) r[m] = 0.5 * (v[va][m] + v[vb][m]);
-  r[4] = 0.25 * (v[0][4] + v[1][4] + v[2][4] + v[3][4]);
-  for (int q = 0; q < 4; q++) {
-    const Block &b = blocks[J[q * 3]];
-    for (int m = 0; m < 5; m++) b.qa[(size_t)m * b.N + lq[q]] = r[m];
-    if (prim) put_primitives(b, coef[b.cs], phys(), lq[q], r);
+  __syncthreads();   // the members' states are read before any is written
+  if (!on) return;
+  const Block &b = blocks[J[q * 3]];
+  const CaseCoef &c = coef[b.cs];
+  const int ip = J[q * 3 + 1], jp = J[q * 3 + 2], i = ip * (b.nx - 1), j = jp * (b.ny - 1);
+  const int l = indx3(b, i, j, k, 0);
+#pragma unroll
+  for (int m = 0; m < 5; m++) b.qa[(size_t)m * b.N + l] = r[m];
+  if (prim) put_primitives(b, c, phys(), l, r);
+  if (cap) {
+    if (avg_face(b, c, 0, ip)) capture_face(b, 0, ip, i, j, k, r);
+    if (avg_face(b, c, 1, jp)) capture_face(b, 1, jp, i, j, k, r);
+    if (k == 0 && avg_face(b, c, 2, 0)) capture_face(b, 2, 0, i, j, k, r);
+    if (k == b.nz - 1 && avg_face(b, c, 2, 1)) capture_face(b, 2, 1, i, j, k, r);
   }
 }
 
 // ---- interface averaging, Main3D.f90:901-952 ----
-__device__ inline bool avg_code(int np) { return np == 30 || np == 35 || np == 45; }
-
 // capture face values into drva (first loop of the reference)
 __global__ void __launch_bounds__(256) k_avg_capture(StageArgs a) {
   const Work w = a.work[xcd_item(blockIdx.x, gridDim.x)];
@@ -1190,12 +1231,6 @@ __device__ inline double avg_count(const Block &b, const CaseCoef &c, int x, int
       }
     }
   return cnt + self_inc;
-}
-
-// whether the interface averaging works on face (d, ip) of block b
-__device__ inline bool avg_face(const Block &b, const CaseCoef &c, int d, int ip) {
-  const int np = b.nbc[d][ip];
-  return avg_code(np) || (c.nextgcic == 1 && (np == 20 || np == 25));
 }
 
 // The reference averages face by face: xi, eta, zeta (the two faces of a
@@ -1479,9 +1514,9 @@ void launch_sc_end(const CaseCoef *coef, double *sc, int ncase, hipStream_t st) 
   hipLaunchKernelGGL(k_sc_end, dim3((ncase + 63) / 64), dim3(64), 0, st, coef, sc, ncase);
 }
 void launch_junction(const Block *blocks, const CaseCoef *coef, const int *jct, const int *jvel, int njct, int maxk,
-                     int prim, hipStream_t st) {
-  int tot = njct * maxk;
-  hipLaunchKernelGGL(k_junction, dim3((tot + 63) / 64), dim3(64), 0, st, blocks, coef, jct, jvel, njct, maxk, prim);
+                     int prim, int cap, hipStream_t st) {
+  const int tot = 4 * njct * maxk;
+  hipLaunchKernelGGL(k_junction, dim3((tot + 63) / 64), dim3(64), 0, st, blocks, coef, jct, jvel, njct, maxk, prim, cap);
 }
 
 }  // namespace tp
