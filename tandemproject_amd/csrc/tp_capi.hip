@@ -993,13 +993,12 @@ void enqueue_begin(tp_context *c, int nk, bool prim_ready = false, bool lean = f
 void enqueue_gradients(tp_context *c) {
   if (!c->any_visc) return;
   const bool dir = direct_ok(c, 0);
-  if (dir && c->L.dirs.P) {
+  // (apart while the derivative class is timed: its counts and bytes are per direction)
+  if (dir && c->L.dirs.P && !(c->prof && (c->prof_mask >> K_DERIV & 1))) {
     const ColGroup &g = c->L.dirs;
-    Timed t(c, K_DERIV, 16.0 * (double)c->npts * 12, true);
     LineArgs a = line_args(c, F_DE, 1, F_FX, 0, 0, 0, 1, 3);
     a.work = g.work.d;
-    hipEvent_t e0 = t.start(0), e1 = t.stop(0, 1);
-    launch_col_dirs(g.C, g.P, g.work.n, 4, c->stream, a, e0, e1);
+    launch_col_dirs(g.C, g.P, g.work.n, 4, c->stream, a);
     return;
   }
   if (!dir) run_exchange(c, 0, 1, 0, F_DE, 1, 4, 1);

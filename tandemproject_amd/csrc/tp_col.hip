@@ -363,11 +363,11 @@ int col_capacity(int chunk) {
 // capacity of a launch of all three directions, at least C
 int dirs_capacity(int C) { return C <= 12 ? 12 : C <= 16 ? 16 : C <= 24 ? 24 : 32; }
 
-void launch_col_dirs(int C, int P, int nwg, int nf, hipStream_t st, const LineArgs &a, hipEvent_t e0, hipEvent_t e1) {
+void launch_col_dirs(int C, int P, int nwg, int nf, hipStream_t st, const LineArgs &a) {
   const size_t lds = col_lds_bytes(0, P, 1);
   switch (C) {
 #define CASE_C(CV) \
-  case CV: TP_LAUNCH_EV((k_col_dirs<CV>), dim3(nwg, nf), dim3(64 * P), lds, st, e0, e1, a); break;
+  case CV: hipLaunchKernelGGL(k_col_dirs<CV>, dim3(nwg, nf), dim3(64 * P), lds, st, a); break;
     CASE_C(12) CASE_C(16) CASE_C(24) CASE_C(32)
 #undef CASE_C
   }

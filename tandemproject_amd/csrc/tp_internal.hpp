@@ -294,8 +294,7 @@ void launch_col(int d, int kind, int C, int P, int G, int nwg, int nf, hipStream
                 hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
 // derivatives along all three directions in one launch (Work::d)
 int dirs_capacity(int C);
-void launch_col_dirs(int C, int P, int nwg, int nf, hipStream_t st, const LineArgs &a, hipEvent_t e0 = nullptr,
-                     hipEvent_t e1 = nullptr);
+void launch_col_dirs(int C, int P, int nwg, int nf, hipStream_t st, const LineArgs &a);
 void launch_deriv(int d, int nwg, int nf, size_t lds, hipStream_t st, const LineArgs &a,
                   hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
 void launch_filter(int d, int nwg, int nf, size_t lds, hipStream_t st, const LineArgs &a,
