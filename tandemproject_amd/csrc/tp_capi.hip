@@ -537,6 +537,9 @@ struct tp_context {
                                    // step k from stage k's update on (set by enqueue_step only)
   bool qin = false;                // kernels enqueued now read the stage's state from qo
                                    // (StageArgs::qin): set by enqueue_step only
+  bool stats = false;              // some case has been asked for surface statistics: the stages
+                                   // enqueue their kernels (two launches that return at once
+                                   // cost a step 4 us at 28 k points, 9 in graph replays)
   int col_fixed = 0;               // requested chunks per line (0: chosen per direction)
   // autotuned chunks per line for each direction, kind and line-length class (-1: none)
   int tuned[3][2][kNClass];
@@ -1010,7 +1013,7 @@ void enqueue_gradients(tp_context *c) {
 // surface forces and pressure statistics, src/Main3D.f90:695-706 (the
 // kernels return at once for cases that do not sample this step)
 void enqueue_surface(tp_context *c, int nk) {
-  if (nk != 1 || !c->L.surf.n) return;
+  if (nk != 1 || !c->stats || !c->L.surf.n) return;
   StageArgs a = base_args(c);
   a.nk = nk;
   run_faces(c, c->L.surf, FK_SURF_SAMPLE, a, K_MISC);
@@ -2776,6 +2779,10 @@ int32_t tp_stats_start(tp_context *c, int32_t cs, int32_t every) {
   double s[S_STRIDE];
   HIPCHK(hipMemcpyAsync(s, c->d_sc + h->slot * S_STRIDE, sizeof(s), hipMemcpyDeviceToHost, c->stream));
   HIPCHK(hipStreamSynchronize(c->stream));
+  if (every > 0 && !c->stats) {
+    drop_graph(c);   // captured without the statistics
+    c->stats = true;
+  }
   s[S_ST_EVERY] = every;
   s[S_ST_T0] = s[S_ST_TP] = s[S_ST_NS] = 0.0;
   s[S_CL] = s[S_CD] = s[S_CLS] = s[S_CDS] = 0.0;
