@@ -237,7 +237,9 @@ int32_t tp_sync(tp_context *ctx);
  *   chunked sweeps for every block and direction whose lines L allow chunks
  *   of ceil(L/P) <= 32 points; 0 (default) lets the library choose per block
  *   and direction.  Lines of 513 to 1024 points are cut into chunks of at most
- *   24 points whatever P is; longer ones run the sequential sweep.  The chunk count of a block depends only on its own line
+ *   24 points whatever P is; longer ones, and filters of such lines with a
+ *   cut-off so sharp that its carries hardly decay (above about 0.96 pi), run the
+ *   sequential sweep.  The chunk count of a block depends only on its own line
  *   lengths (and on the autotuner's choice for its line-length class), so a
  *   case computes bit-identical results alone or batched with others when
  *   the chunk counts are fixed or left at their defaults.

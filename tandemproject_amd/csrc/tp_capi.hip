@@ -357,7 +357,7 @@ size_t col_table_doubles(int L, int P) {
 }
 
 // Waves of the line solves of a line longer than 16 chunks hold (512 points),
-// up to COL_LONG_MAX points; 0 for other lines.  They take COL_LONG_G chunks in
+// up to COL_LONG_MAX points; 0 for other lines (and see block_waves).  They take COL_LONG_G chunks in
 // each wave, the fewest waves of full chunks (k_col).  701-point xi lines,
 // 1.3 M points, a launch of 4.5 fields on average: sequential 310 us, 16 waves
 // of 11-point chunks 79, 11 of 16 71, 8 of 22 54.  Up to 512 points one chunk a
@@ -372,6 +372,43 @@ int long_chunk(int L) { return (L + COL_LONG_G * long_waves(L) - 1) / (COL_LONG_
 size_t long_table_doubles(int L) {
   const int Cl = long_chunk(L), Pe = (L + Cl - 1) / Cl;
   return (8 * COL_LONG_Q + (size_t)COL_LONG_F * Pe + 15) / 16 * 16;
+}
+
+// Chunks that a carry crosses before it has died out: the fewest w for which
+// the maps of any w chunks in a row, forwards and backwards, leave at most
+// 1e-20 of it, so that even a carry 1e4 times the values it enters stays below
+// their rounding.  From the long table T itself, since the decay is the
+// scheme's: 0.74 a point for the derivative, for the filter 0.72 at a cut-off
+// of 0.85 pi, 0.90 at 0.95, 0.98 at 0.99 (8, 7, 20 and more than COL_LONG_R
+// chunks of 22 points).  0 where COL_LONG_R chunks do not reach it (and for
+// factors that are not finite): the sequential kernel, exact for any factors.
+int long_reach(const std::vector<double> &T, int L) {
+  const int Cl = long_chunk(L), Pe = (L + Cl - 1) / Cl;
+  // m (from the left) times p
+  auto times = [](const double *m, const double p[4], double o[4]) {
+    for (int i = 0; i < 2; i++)
+      for (int j = 0; j < 2; j++) o[2 * i + j] = m[2 * i] * p[j] + m[2 * i + 1] * p[2 + j];
+  };
+  auto small = [](const double p[4]) {
+    bool s = true;
+    for (int i = 0; i < 4; i++) s = s && std::fabs(p[i]) <= 1e-20;   // false for NaN
+    return s;
+  };
+  for (int w = 1; w <= std::min(COL_LONG_R, Pe - 1); w++) {
+    bool dead = true;
+    for (int q = 0; q + w <= Pe && dead; q++) {
+      double f[4] = {1, 0, 0, 1}, g[4] = {1, 0, 0, 1}, t[4];
+      for (int k = 0; k < w; k++) {
+        times(&T[4 * (q + k)], f, t);
+        std::copy(t, t + 4, f);
+        times(&T[4 * COL_LONG_Q + 4 * (q + w - 1 - k)], g, t);
+        std::copy(t, t + 4, g);
+      }
+      dead = small(f) && small(g);
+    }
+    if (dead) return w;
+  }
+  return 0;
 }
 
 // doubles of all chunked-solver tables of a block with lines L[3]: every
@@ -743,6 +780,10 @@ void drop_graph(tp_context *c) {
 
 int block_default(const Block &b, int d) { return col_default(b.L[d], b.ndf[d][0] || b.ndf[d][1]); }
 
+// waves of block b's line solves in the long-line layout, 0 if they have
+// another: lines of another length, or a filter whose carries decay too slowly
+int block_waves(const Block &b, int d, int kind) { return b.colR[d][kind] ? long_waves(b.L[d]) : 0; }
+
 // chunks per line of block g's line solves in direction d, kind: the tuned
 // count of its line-length class if that fits its lines, else the requested
 // count if it fits, else the default (0: the sequential kernel)
@@ -763,7 +804,7 @@ void choose_lines(tp_context *c) {
     const auto &src = c->bsrc[g];
     for (int d = 0; d < 3; d++)
       for (int kind = 0; kind < 2; kind++) {
-        const int P = block_chunks(c, (int)g, d, kind), W = long_waves(c->blocks[g].L[d]);
+        const int P = block_chunks(c, (int)g, d, kind), W = block_waves(c->blocks[g], d, kind);
         const int ci = W ? 0 : col_class(P) - 1;
         c->blocks[g].colP[d][kind] = W ? W : P;
         c->blocks[g].col[d][kind] =
@@ -826,7 +867,7 @@ int make_groups(tp_context *c, const std::vector<int> &gs, Mem &m, ListSet &L) {
       std::vector<std::vector<Work>> works;
       for (int g : gs) {
         const Block &b = c->blocks[g];
-        const int W = long_waves(b.L[d]), G = W ? COL_LONG_G : 1;
+        const int W = block_waves(b, d, kind), G = W ? COL_LONG_G : 1;
         const int P = W ? W : block_chunks(c, g, d, kind);
         const int C = W ? COL_LONG_C : P ? col_capacity((b.L[d] + P - 1) / P) : 0;
         // a chunked launch reads the block's carry-map and factor table
@@ -914,7 +955,7 @@ int make_groups(tp_context *c, const std::vector<int> &gs, Mem &m, ListSet &L) {
 // the chunk count that covers the most points (0: the sequential kernel)
 int top_chunks(const tp_context *c, int d, int kind) {
   long long n[17] = {0};
-  for (const Block &b : c->blocks) n[long_waves(b.L[d]) ? 0 : b.colP[d][kind]] += b.N;
+  for (const Block &b : c->blocks) n[block_waves(b, d, kind) ? 0 : b.colP[d][kind]] += b.N;
   return (int)(std::max_element(n, n + 17) - n);
 }
 
@@ -1462,6 +1503,7 @@ int build_case(HostCase &h) {
           const std::vector<double> &lu = kind == 0 ? lud : luf;
           std::vector<double> T = col_tables(L, COL_LONG_G * long_waves(L), &lu[0 * nl + o], &lu[1 * nl + o],
                                              &lu[2 * nl + o], &lu[3 * nl + o], &lu[4 * nl + o], true);
+          b.colR[d][kind] = long_reach(T, L);
           slot.push_back({(d * 2 + kind) * kNColP, all.size()});
           T.resize(long_table_doubles(L), 0.0);
           all.insert(all.end(), T.begin(), T.end());

@@ -191,7 +191,6 @@ __device__ inline double filter_bnd_row(const Block &b, const CaseCoef &c, int D
 
 
 constexpr int COL_TR = 65;   // row pitch (doubles) of the xi transpose buffer
-constexpr int COL_REACH = 160;  // points beyond which a carry has died out (long lines)
 constexpr int COL_DECAY = 48;  // points a carry travels sequentially before an amplifying closure
 
 // doubles of one chunk's factors in LDS: the table's own [6][32], or a long

@@ -35,9 +35,9 @@
   double *tr = reinterpret_cast<double *>(pairB + PL * 64) + PL * G * FC + wv * (8 * COL_TR);
   const double *T = b.col[D][KIND];
   // carry maps: of all chunks (G = 1), or of the window of chunks that this
-  // wave composes: a carry decays by 0.74 per point, so what comes from more
-  // than COL_REACH points away is below 1e-20 of it
-  const int reach = G == 1 ? 0 : (COL_REACH + Cl - 1) / Cl;
+  // wave composes: what comes from further away has died out (long_reach forms
+  // the distance from the block's own factors; it depends on the filter's cut-off)
+  const int reach = G == 1 ? 0 : b.colR[D][KIND];
   const int qf0 = G == 1 ? 0 : max(0, wv * G - reach), qb0 = G == 1 ? 0 : wv * G;
   double mapf[G == 1 ? 1 : 2], mapb[G == 1 ? 1 : 2];
   if (G == 1) {
@@ -194,7 +194,19 @@
   // in by the (at most two) chunks at each end that hold them; then the
   // padding rows zeroed
   double r[C];
-  if (KIND == 1) {
+  if (KIND == 1 && G > 1) {
+    // long lines: the increment, added to the input at the store, as the
+    // sequential kernel forms it.  A out = R + A in (below) reads the input
+    // once, but its rounding grows with A's condition: 3.5e-14 of the field
+    // at a cut-off of 0.85 pi, 1.6e-12 at 0.95, where the increment keeps
+    // 1.1e-16 and 1.2e-16
+#pragma unroll
+    for (int k = 0; k < C; k++) {
+      const double res = 2.0 * v[k + 3];
+      r[k] = c.fa * (v[k + 2] + v[k + 4] - res) + c.fb * (v[k + 1] + v[k + 5] - res) +
+             c.fc * (v[k] + v[k + 6] - res);
+    }
+  } else if (KIND == 1) {
     // filter: the solve yields the filtered field itself, A out = R + A in
     // (A the filter's left-hand side: interior rows (fbe, fal, 1, fal, fbe),
     // closure rows of each end from flhs, mirrored at the far end), rather
@@ -339,9 +351,10 @@
     }
   }
 
-  // ---- store: the filtered field, or the derivative (which may accumulate) ----
-  const bool add = KIND == 0 && a.acc;
-  const double *ob = dst;
+  // ---- store: the filtered field (on long lines the input and its increment),
+  // or the derivative (which may accumulate) ----
+  const bool add = KIND == 0 ? a.acc : G > 1;
+  const double *ob = KIND == 0 ? dst : src;
   double *cpy = KIND == 1 && a.copy_arr >= 0 ? field_ptr(b, a.copy_arr, a.copy_col + fi * a.out_step) : nullptr;
   // xi: the work item's lines are consecutive rows of the block, one
   // contiguous span of nl * L doubles.  Once every wave is done with the

@@ -26,6 +26,9 @@ constexpr int MAX_CASE = 4096;
 // chunk's factors, padded so that the lane groups' reads of one row fall into
 // different LDS banks (2 x 120 = 48 modulo the 64 banks)
 constexpr int COL_LONG_G = 4, COL_LONG_C = 24, COL_LONG_Q = 44, COL_LONG_MAX = 1024, COL_LONG_F = 120;
+// most chunks before (after) its own that a wave composes: with its own they
+// are the 32 whose maps two registers hold
+constexpr int COL_LONG_R = 32 - COL_LONG_G;
 constexpr int RCV_SLOTS = 5;  // fields whose closure sums one exchange launch can hold
 
 // ---- per-case scalars on the device (src/MainVar3D.f90:139-142) ----
@@ -106,6 +109,8 @@ struct Block {
   const double *col[3][2];    // chunked-solver carry maps per direction, kind (deriv, filter)
   int colP[3][2];             // chunks per line they are for (0: the sequential kernel); in the
                               // long-line layout waves, COL_LONG_G chunks each
+  int colR[3][2];             // long lines: chunks that a carry crosses before it has died out, at
+                              // most COL_LONG_R (0: not in the long-line layout)
 };
 
 // array ids exposed through the C ABI (order shared with include/tandem_hip.h)
