@@ -574,9 +574,10 @@ struct tp_context {
                                    // step k from stage k's update on (set by enqueue_step only)
   bool qin = false;                // kernels enqueued now read the stage's state from qo
                                    // (StageArgs::qin): set by enqueue_step only
-  bool stats = false;              // some case has been asked for surface statistics: the stages
-                                   // enqueue their kernels (two launches that return at once
-                                   // cost a step 4 us at 28 k points, 9 in graph replays)
+  bool stats = false;              // some linked case samples surface statistics (its S_ST_EVERY > 0;
+                                   // set by link and tp_stats_start): the stages enqueue their kernels
+                                   // (two launches that return at once cost a step 4 us at 28 k points,
+                                   // 9 in graph replays)
   int col_fixed = 0;               // requested chunks per line (0: chosen per direction)
   // autotuned chunks per line for each direction, kind and line-length class (-1: none)
   int tuned[3][2][kNClass];
@@ -1613,7 +1614,7 @@ int link(tp_context *c) {
   c->d_wr = nullptr; c->d_wwr = nullptr; c->d_jct = nullptr; c->d_jvel = nullptr;
   c->L = ListSet();
   c->blocks.clear(); c->bsrc.clear(); c->linked.clear();
-  c->npts = 0; c->any_visc = false; c->njct = 0; c->maxk = 0;
+  c->npts = 0; c->any_visc = false; c->stats = false; c->njct = 0; c->maxk = 0;
   std::vector<CaseCoef> coefs;
   std::vector<double> sc;
   for (size_t i = 0; i < c->cases.size(); i++) {
@@ -1626,6 +1627,7 @@ int link(tp_context *c) {
     coefs.push_back(h.coef);
     if (h.sc_saved) {
       sc.insert(sc.end(), h.sc, h.sc + S_STRIDE);
+      if (h.sc[S_ST_EVERY] > 0) c->stats = true;   // the case went on sampling, here or where it came from
     } else {
       sc.insert(sc.end(), S_STRIDE, 0.0);
       sc[h.slot * S_STRIDE + S_AOA] = h.dp[TP_D_AOA0];
