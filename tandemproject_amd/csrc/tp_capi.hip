@@ -489,6 +489,13 @@ struct Mem {
     p.clear();
     bytes = 0;
   }
+  // take over another owner's allocations
+  void take(Mem &o) {
+    p.insert(p.end(), o.p.begin(), o.p.end());
+    bytes += o.bytes;
+    o.p.clear();
+    o.bytes = 0;
+  }
 };
 
 // chunked-solver tables of one block: direction x kind x chunk-count index
@@ -582,6 +589,8 @@ struct tp_context {
   // autotuned chunks per line for each direction, kind and line-length class (-1: none)
   int tuned[3][2][kNClass];
   Mem lmem;                        // line-solve launch tables (rebuilt when the chunk choice changes)
+  bool hold = false;               // launch tables and work areas no longer used go to held, not to
+  Mem held;                        // hipFree, until tp_destroy (hold_frees)
   long long npts = 0;
   bool any_visc = false;
   // measurement
@@ -620,6 +629,12 @@ int upload_vec(Mem &m, T **dptr, const std::vector<T> &v) {
   if (rc) return rc;
   if (!v.empty()) HIPCHK(hipMemcpy(*dptr, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice));
   return 0;
+}
+
+// free a context's launch tables or a work area, or hold them (hold_frees)
+void give_back(tp_context *c, Mem &m) {
+  if (c->hold) c->held.take(m);
+  else m.release();
 }
 
 int upload_list(Mem &m, DevList &L, const std::vector<Work> &v) {
@@ -966,7 +981,7 @@ int regroup(tp_context *c) {
   drop_graph(c);
   HIPCHK(hipStreamSynchronize(c->stream));
   choose_lines(c);
-  c->lmem.release();
+  give_back(c, c->lmem);
   std::vector<int> gs(c->blocks.size());
   for (size_t g = 0; g < gs.size(); g++) gs[g] = (int)g;
   if (int rc = make_groups(c, gs, c->lmem, c->L)) return rc;
@@ -1608,8 +1623,8 @@ int link(tp_context *c) {
     }
   }
   drop_graph(c);
-  c->link.release();
-  c->lmem.release();
+  give_back(c, c->link);
+  give_back(c, c->lmem);
   c->d_blocks = nullptr; c->d_coef = nullptr; c->d_sc = nullptr; c->d_part = nullptr; c->d_wpart = nullptr;
   c->d_wr = nullptr; c->d_wwr = nullptr; c->d_jct = nullptr; c->d_jvel = nullptr;
   c->L = ListSet();
@@ -1711,6 +1726,10 @@ void gust_mode(double tu, double kr, const double *u, double *m8, double *slit) 
 }
 
 }  // namespace
+
+namespace tp {
+void hold_frees(tp_context *c) { c->hold = true; }
+}  // namespace tp
 
 // ----------------------------------------------------------------------------
 // C ABI
@@ -1894,6 +1913,7 @@ int32_t tp_destroy(tp_context *c) {
   for (auto &h : c->cases) h.mem.release();
   c->link.release();
   c->lmem.release();
+  c->held.release();
   (void)hipStreamDestroy(c->stream);
   delete c;
   return 0;
@@ -2113,7 +2133,7 @@ int32_t tp_setup_geometry(tp_context *c) {
     ListSet sub;
     int rc = make_lists(c, gs, tmp, sub);
     if (!rc) rc = make_groups(c, gs, tmp, sub);
-    if (rc) { tmp.release(); return rc; }
+    if (rc) { give_back(c, tmp); return rc; }
     std::swap(c->L, sub);
     const int dst[3] = {F_QO, F_QA, F_DE};
     for (int m = 0; m < 3; m++) {
@@ -2127,7 +2147,7 @@ int32_t tp_setup_geometry(tp_context *c) {
     run_faces(c, c->L.surf, FK_SURF_SETUP, base_args(c), K_MISC);
     std::swap(c->L, sub);
     const hipError_t e = hipStreamSynchronize(c->stream);
-    tmp.release();
+    give_back(c, tmp);
     if (e != hipSuccess) return fail(TP_E_HIP, std::string("metrics: ") + hipGetErrorString(e));
   }
   // wall-slot flags (SingleTurbulence3D.f90:447-464), sponge coefficients
@@ -2241,13 +2261,13 @@ int32_t tp_setup_geometry(tp_context *c) {
             Mem tmp;
             double *ded = nullptr, *dpos = nullptr;
             if ((rc = upload_vec(tmp, &ded, h.eddies)) || (rc = upload_vec(tmp, &dpos, pos))) {
-              tmp.release();
+              give_back(c, tmp);
               return rc;
             }
             launch_eddy_table(ded, (int)(h.eddies.size() / 10), dpos, b.ngust, h.coef.ntz, h.coef.fctr, h.coef.uoo,
                               h.dp[TP_D_SLIT], h.dp[TP_D_SPAN], h.dp[TP_D_CFIT], b.vito, c->stream);
             const hipError_t e = hipStreamSynchronize(c->stream);
-            tmp.release();
+            give_back(c, tmp);
             if (e != hipSuccess) return fail(TP_E_HIP, std::string("eddy table: ") + hipGetErrorString(e));
             HIPCHK(hipGetLastError());
             continue;   // what follows builds the Fourier-mode table of inflow 1 and 2
@@ -2278,13 +2298,13 @@ int32_t tp_setup_geometry(tp_context *c) {
           double *dmodes = nullptr, *dpos = nullptr, *drot = nullptr;
           if ((rc = upload_vec(tmp, &dmodes, modes)) || (rc = upload_vec(tmp, &dpos, pos)) ||
               (rc = upload_vec(tmp, &drot, rot))) {
-            tmp.release();
+            give_back(c, tmp);
             return rc;
           }
           launch_inflow_table(dmodes, drot, nm, dpos, b.ngust, h.coef.ntz, h.coef.fctr, h.coef.uoo, b.vito,
                               c->stream);
           const hipError_t e = hipStreamSynchronize(c->stream);
-          tmp.release();
+          give_back(c, tmp);
           if (e != hipSuccess) return fail(TP_E_HIP, std::string("inflow table: ") + hipGetErrorString(e));
           HIPCHK(hipGetLastError());
         }

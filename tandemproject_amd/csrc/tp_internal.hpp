@@ -14,6 +14,8 @@
 #include <string>
 #include <vector>
 
+struct tp_context;
+
 namespace tp {
 
 constexpr int LMD = 11;   // deriv closure length - 1 (src/MainVar3D.f90:19)
@@ -327,6 +329,14 @@ void launch_surf_reduce(const CaseCoef *coef, double *sc, const double *wpart, c
 
 // host: record the message of a failure (tp_last_error) and return its code
 int set_error(int code, const std::string &msg);
+// host: from now on the context keeps the launch tables and work areas that it
+// is done with until tp_destroy.  hipFree waits until every stream of the device
+// is idle: while other contexts step, each of the some hundred small frees of a
+// case's set-up waited for the steps enqueued then (24 of them 940 ms beside
+// 20 M points), so that requests were not set up before the running case ended.
+// A set-up keeps its launch tables (below 1 MB) and 24 B an inflow point that way.
+// A case's own memory is freed at once as ever.
+void hold_frees(tp_context *c);
 
 enum PointKernel { PK_PRIM = 0, PK_DTRED, PK_FORCE = 5, PK_SPONGE = 6, PK_RK, PK_RK_PRIM, PK_COPYF = 9, PK_INIT, PK_METRICS,
                    PK_FLUXALL = 14, PK_STRESS = 15, PK_FLUX_TV = 16 };

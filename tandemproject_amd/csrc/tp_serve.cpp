@@ -4,9 +4,10 @@
 // while others join and leave (continuous batching), and leave the device
 // with their final state copied to the host.  Set-up runs on a staging
 // thread, each request in a context (and stream) of its own, beside the
-// stepping of the resident cases; a set-up case joins them between steps
-// without a copy (tp_adopt_cases).  Host code over the C ABI only; the
-// device work is the contexts'.  No counterpart in the reference, which runs
+// stepping of the resident cases (their contexts free nothing then:
+// hold_frees); a set-up case joins them between steps without a copy
+// (tp_adopt_cases).  Host code over the C ABI otherwise; the device work is
+// the contexts'.  No counterpart in the reference, which runs
 // one case per MPI job.
 #include <hip/hip_runtime.h>
 
@@ -25,6 +26,7 @@
 #include <vector>
 
 #include "../../include/tandem_hip.h"
+#include "tp_internal.hpp"
 
 namespace {
 
@@ -527,6 +529,7 @@ int32_t tp_server_submit(tp_server *s, int32_t nblocks, const int32_t *dims, con
   std::shared_lock<std::shared_mutex> hl(s->hip_mu);
   Request q;
   if (int rc = tp_create(&q.sctx)) return srv_fail(s, rc, tp_last_error());
+  tp::hold_frees(q.sctx);
   auto drop = [&](int rc, const std::string &m) {
     tp_destroy(q.sctx);
     return srv_fail(s, rc, m);
