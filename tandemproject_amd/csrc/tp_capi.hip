@@ -2980,6 +2980,9 @@ int32_t tp_case_params(tp_context *c, int32_t cs, int32_t *iparams, double *dpar
 // ---- the derivative of one field held by the caller ----
 namespace {
 
+// bytes of the work area that tp_field_deriv_noalloc takes its calls' from
+constexpr size_t kScratchBytes = (size_t)1 << 20;
+
 // device bytes of the work area of tp_field_deriv: block view, coefficients,
 // chunked-solver table, work list (each 256-byte aligned)
 struct FieldWs {
@@ -3032,7 +3035,13 @@ int field_prepare(int32_t lxi, int32_t let, int32_t lze, const int32_t *nbc2, in
   f.periodic = nbc2[0] == 45;
   if (f.L < (f.periodic ? LMD + 2 : 7))
     return fail(TP_E_LAYOUT, "tp_field_deriv: lines of " + std::to_string(f.L) + " points are too short");
+  const int64_t nlines = np / f.L, nwork = (nlines + 63) / 64;
   f.P = col_default(f.L, f.periodic);
+  // a call of nearly as many lines as fit the work area with tables of half as
+  // many chunks takes those (here, so that the two entries give the same bits)
+  if (f.P > 1 && col_chunk(f.L, f.P / 2) && field_ws(f.L, f.P, (int)nwork).total > kScratchBytes &&
+      field_ws(f.L, f.P / 2, (int)nwork).total <= kScratchBytes)
+    f.P /= 2;
   if (!f.P) return fail(TP_E_SIZE, "tp_field_deriv: lines longer than 512 points need a context (tp_deriv)");
   f.C = col_capacity((f.L + f.P - 1) / f.P);
   std::memset(&f.blk, 0, sizeof(Block));
@@ -3066,7 +3075,6 @@ int field_prepare(int32_t lxi, int32_t let, int32_t lze, const int32_t *nbc2, in
   const int end = f.periodic ? 1 : 0;
   band_lu(f.L, albed[end], albed[end], kAlpha, kBeta, l1, l2, u1, u2, u3);
   f.tab = col_tables(f.L, f.P, l1, l2, u1, u2, u3);
-  const int64_t nlines = np / f.L;
   f.work.clear();
   for (int64_t q = 0; q < nlines; q += 64) f.work.push_back({0, (int)q, (int)std::min<int64_t>(64, nlines - q), d});
   f.nwork = (int)f.work.size();
@@ -3121,7 +3129,6 @@ int32_t tp_field_deriv(int32_t lxi, int32_t let, int32_t lze, const int32_t *nbc
 // call on each device.  Calls that overlap on one GPU (other streams, other
 // host threads) share it and race; calls in turn on one stream are ordered.
 // Nothing in it needs to start at zero: every call writes the parts it reads.
-constexpr size_t kScratchBytes = (size_t)1 << 20;
 static __device__ __align__(256) char scratch[kScratchBytes];
 
 namespace {
