@@ -455,7 +455,10 @@ int32_t tp_server_set_staging(tp_server *srv, int32_t ahead);
 /* admit no further request while the cases on the device hold at least
  * `points` grid points (one case is always admitted; 0: no limit, the
  * default).  Enough points to fill the GPU keep its throughput while large
- * cases finish one after another instead of sharing it. */
+ * cases finish one after another instead of sharing it: while the device holds
+ * at least half of `points`, a request that would take it past them waits, and
+ * later ones that fit go first as long as their work (points times steps) stays
+ * within an eighth of its own. */
 int32_t tp_server_set_fill(tp_server *srv, int64_t points);
 /* message of the last failed server call on the calling thread */
 const char *tp_server_error(tp_server *srv);
