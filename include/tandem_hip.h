@@ -240,8 +240,8 @@ int32_t tp_sync(tp_context *ctx);
  *   24 points whatever P is; longer ones, and filters of such lines with a
  *   cut-off so sharp that its carries hardly decay (above about 0.96 pi), run the
  *   sequential sweep.  The chunk count of a block depends only on its own line
- *   lengths (and on the autotuner's choice for its line-length class), so a
- *   case computes bit-identical results alone or batched with others when
+ *   lengths and end types (closure or one-sided; and on the autotuner's choice
+ *   for its class of lines), so a case computes bit-identical results alone or batched with others when
  *   the chunk counts are fixed or left at their defaults.
  * TP_OPT_STRESSES = 1: every stage leaves the viscous stresses and heat
  *   fluxes (the reference's txx, tyy, tzz, txy, tyz, tzx, hxx, hyy, hzz) in

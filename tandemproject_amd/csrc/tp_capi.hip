@@ -382,6 +382,8 @@ size_t long_table_doubles(int L) {
 // of 0.85 pi, 0.90 at 0.95, 0.98 at 0.99 (8, 7, 20 and more than COL_LONG_R
 // chunks of 22 points).  0 where COL_LONG_R chunks do not reach it (and for
 // factors that are not finite): the sequential kernel, exact for any factors.
+// (An infinity or NaN on a line reaches the chunks within that distance, where
+// the sequential sweep spreads it over the whole line.)
 int long_reach(const std::vector<double> &T, int L) {
   const int Cl = long_chunk(L), Pe = (L + Cl - 1) / Cl;
   // m (from the left) times p

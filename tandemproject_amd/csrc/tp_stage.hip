@@ -1239,7 +1239,7 @@ __device__ inline double avg_count(const Block &b, const CaseCoef &c, int x, int
 // thread of the point's first averaged face carries it through the others in
 // turn, the threads of the others leave it alone.  (Three launches took 16-17 us a
 // stage at 28 k and 208 k points, one, with the copy to drvb, 7-8 us; 54 and
-// 40 us at 20 M points.)
+// 47 us at 20 M points.)
 __global__ void __launch_bounds__(256) k_avg_apply(StageArgs a) {
   const Work w = a.work[xcd_item(blockIdx.x, gridDim.x)];
   const Block &b = a.blocks[w.blk];
